@@ -1069,16 +1069,26 @@ static void skinny_launch(const GemmArgs &a, float *ws, size_t ws_bytes, hipStre
     launch_reduce<EPI, NB>(a, ws, splits, s);
 }
 
+static void init_cus() {
+    if (g_cus) return;
+    int dev = 0;
+    ESP_HIP(hipGetDevice(&dev));
+    ESP_HIP(hipDeviceGetAttribute(&g_cus, hipDeviceAttributeMultiprocessorCount, dev));
+    if (g_cus <= 0) g_cus = 256;
+}
+
+void launch_gemm_reduce(GemmEpi epi, const GemmArgs &a, const float *ws, int splits, hipStream_t s) {
+    init_cus();
+    if (epi == GEMM_STORE) launch_reduce<GEMM_STORE, 1>(a, ws, splits, s);
+    else if (epi == GEMM_RESIDUAL) launch_reduce<GEMM_RESIDUAL, 1>(a, ws, splits, s);
+    else launch_reduce<GEMM_SWIGLU, 2>(a, ws, splits, s);
+}
+
 template <int EPI> static void mfma_launch(const GemmArgs &a, float *ws, size_t ws_bytes,
                                            hipStream_t s) {
     constexpr int NB = EPI == GEMM_SWIGLU ? 2 : 1;
     constexpr int NJW = 4 / NB;  // wide form: 128 weight columns per wave
-    if (!g_cus) {
-        int dev = 0;
-        ESP_HIP(hipGetDevice(&dev));
-        ESP_HIP(hipDeviceGetAttribute(&g_cus, hipDeviceAttributeMultiprocessorCount, dev));
-        if (g_cus <= 0) g_cus = 256;
-    }
+    init_cus();
     const long long wide_tiles = (long long)((a.N + 64 * NJW - 1) / (64 * NJW)) * ((a.M + MF_BM - 1) / MF_BM);
     // long row counts (prefill of >= 1024 tokens) take the LDS-streamed form:
     // 256-row blocks for one weight matrix, 128-row blocks for gate/up pairs

@@ -1,6 +1,6 @@
 // Generic tiled projection GEMM, C[M,N] = A[M,K] . W[N,K]^T with f32
-// accumulation on the vector ALUs. It serves the f32 weight format (where
-// every product must stay f32) and shapes the MFMA kernel does not tile.
+// accumulation on the vector ALUs. It serves the shapes that the matrix-core
+// kernels do not tile (K no multiple of 16, unaligned operands).
 #include "common.hpp"
 #include "dev.hpp"
 

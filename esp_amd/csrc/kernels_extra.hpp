@@ -15,6 +15,9 @@ void launch_fill_const(float *dst, size_t n, float v, hipStream_t s);
 void launch_fill_bits(uint16_t *dst, size_t n, uint16_t bits, hipStream_t s);
 
 void launch_gemm_simple(Dt wt, GemmEpi epi, const GemmArgs &a, hipStream_t s);
+// The sums of a GEMM's `splits` k-split partials ([splits][matrices][M][N]
+// f32 at ws, in split order), then the epilogue.
+void launch_gemm_reduce(GemmEpi epi, const GemmArgs &a, const float *ws, int splits, hipStream_t s);
 
 // moe.rs:156-181 routing on the device.
 struct RouteArgs {

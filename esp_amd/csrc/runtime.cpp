@@ -1129,7 +1129,7 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
         }
     };
     // Split-K partial sums are consumed by the kernel that follows the
-    // projection when it can take them (bf16 activations): the q/k/v sums by
+    // projection when it can take them: the q/k/v sums by
     // the rotary/KV kernel, the o_proj and down_proj residual sums by a row
     // kernel that also applies the next RMSNorm (post-attention, or the next
     // resident layer's input norm: `pre_normed`).
@@ -1177,7 +1177,7 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             g.N = w.qkv_rows;
             g.K = H;
             g.ldc = w.qkv_rows;
-            if (act == DT_SPLIT && rope_kv_fusable(lora_dt(m.wt), kv.dt, m.hd, m.nq, m.nkv, lora_any))
+            if (rope_kv_fusable(lora_dt(m.wt), kv.dt, m.hd, m.nq, m.nkv, lora_any))
                 g.defer_splits = &qkv_splits;
             Prof p("gemm_qkv", s);
             widen_k(m, kv, g);
@@ -1311,7 +1311,7 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             g.N = H;
             g.K = m.qw;
             g.ldc = H;
-            if (!w.moe && act == DT_SPLIT && resid_norm_ok(H)) g.defer_splits = &o_splits;
+            if (!w.moe && resid_norm_ok(H)) g.defer_splits = &o_splits;
             Prof p("gemm_o", s);
             widen_k(m, kv, g);
             launch_gemm(layer_gemm_dt(m.wt), GEMM_RESIDUAL, g, s);
@@ -1382,7 +1382,7 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             d.ldc = H;
             // the next resident layer's input norm takes the partial sums
             int d_splits = 0;
-            const bool next_norm = l + 1 < m.L && !m.st && act == DT_SPLIT && resid_norm_ok(H);
+            const bool next_norm = l + 1 < m.L && !m.st && resid_norm_ok(H);
             if (next_norm) d.defer_splits = &d_splits;
             {
                 Prof p("gemm_down", s);
@@ -1414,8 +1414,14 @@ static void ensure_scratch(Model &m, Kv &kv, int Mc, int n_seqs) {
     kv.last_h.ensure((size_t)n_seqs * H * 4);
     kv.logits.ensure((size_t)std::max(n_seqs, kv.batch) * m.V * 4);
     kv.rows_dev.ensure((size_t)(4 * kMaxRows + 2 * kv.batch + 64) * 4);
-    if (Mc > 1 && (m.wt == DT_BF16 || dt_packed(m.wt)))
-        kv.gemm_ws.ensure((size_t)256 << 20);  // split-K partials
+    if (Mc > 1 && m.wt != DT_F32) kv.gemm_ws.ensure((size_t)256 << 20);  // split-K partials
+    if (Mc > 1 && m.wt == DT_F32) {
+        // the f32 GEMM's partials: splits keep at least 256 keys
+        const size_t kmax = std::max(fmax, std::max(m.H, m.qw));
+        const size_t nmax = std::max(std::max(qkv_rows, m.V), std::max(2 * fmax, m.H));
+        const size_t rows = (size_t)Mc * (m.E ? m.topk : 1);
+        kv.gemm_ws.ensure(std::min<size_t>((size_t)256 << 20, (kmax / 256 + 1) * rows * nmax * 4));
+    }
     if (m.E && !kv.moe_err.p) {
         kv.moe_err.ensure(64);
         launch_fill_const(kv.moe_err.as<float>(), 16, 0.f, kv.stream);

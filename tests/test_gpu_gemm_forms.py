@@ -1,0 +1,38 @@
+"""Projection GEMM forms at the edges of their tiles, against the oracle.
+
+Each case evaluates B one-token sequences in one pass: every projection and
+the head multiply B rows, and every row's logits come back. A one-token
+sequence attends to itself only, so the oracle evaluates each id once.
+"""
+import numpy as np
+import pytest
+
+from esp_amd import DecoderModel
+from oracle import oracle, st
+from tests import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows_match(model, ref, vocab, rows, tol):
+    ids = synth.uniform_ids(rows * 7 + 1, rows, min(vocab, 24))  # few ids: few oracle passes
+    kv = model.new_cache(rows, 4)
+    got = model.forward_batch(kv, list(range(rows)), [[t] for t in ids])
+    want = {t: ref.forward_last(ref.new_cache(), [t]) for t in set(ids)}
+    for r, t in enumerate(ids):
+        scale = float(np.abs(want[t]).max())
+        err = float(np.abs(got[r] - want[t]).max())
+        assert err <= tol * scale, f"row {r} of {rows}: {err} vs scale {scale}"
+
+
+# K of 16-key stages: one stage short of a power of two, k splits (K >= 512),
+# a ragged last split (1040 = 2 x 520), and 72, which keeps the vector form
+@pytest.mark.parametrize("hidden,ffn", [(48, 80), (64, 72), (512, 1040)])
+@pytest.mark.parametrize("rows", [2, 31, 32, 33, 64, 65, 129, 513])
+def test_f32_rows(hidden, ffn, rows):
+    """f32 products and sums: the f32 contract's 1e-4 of the row's magnitude
+    (K 2^-24 is 6e-5 at K 1040 if every rounding went the same way)."""
+    print(f"f32 rows {rows} hidden {hidden} ffn {ffn}", flush=True)
+    cfg, tensors, blob, _ = synth.tiny_llama_case(seed=5, layers=2, hidden=hidden, heads=hidden // 16,
+                                                  kv_heads=hidden // 16, ffn=ffn, vocab=131, prompt_len=2)
+    _rows_match(DecoderModel.from_bytes(cfg, blob, "f32"), oracle.OracleModel(cfg, tensors), 131, rows, 1e-4)
