@@ -119,12 +119,9 @@ struct GemmArgs {
     // them, in split order); a launch without splits applies the epilogue and
     // stores 0.
     int *defer_splits;
-    // Doubled-K packed form (0 = off; the streamed GEMM of >= 1024 rows
-    // only): the weights are [N, K] rows [hi | lo] with K = 2 kdup, the A
-    // planes stay [M, kdup] and are read again for keys kdup .. K, and the
-    // lo plane multiplies only keys below kdup, so the products are
-    // a_hi w_hi + a_lo w_hi + a_hi w_lo without a widened copy of A.
-    int kdup;
+    // Packed weights (DT_Q8 / DT_Q4): the f32 block scales [N, K / 32] of w
+    // and w2.
+    const float *w_scale, *w2_scale;
     // Tile order of the streamed GEMM (set by its launcher): the XCD-major
     // tile ranges walk bands of this many weight-column tiles, row tiles
     // within a band (1 = column-major).
@@ -198,16 +195,6 @@ void launch_pick_fixed(int device, const float *logits, int n, int V, const uint
                        esp_sampler *samplers_dev, uint32_t *ids_dev, uint8_t *flags_dev,
                        hipStream_t s);
 
-// Packed weights: out[i] = q_i * scale[i / 32] in f32 (n a multiple of 32).
-// Packed [N, K] -> bf16 [N, 2K] rows [hi(q*scale) | lo(q*scale)], and split
-// activation planes [M, K] -> [M, 2K] ([hi | hi], [lo | 0]): the doubled-K
-// form of a packed projection for the bf16 matrix-core GEMM.
-void launch_dequant_split(Dt wt, const void *values, const float *scales, size_t N, size_t K,
-                          uint16_t *out, hipStream_t s);
-void launch_widen_split(const uint16_t *hi, const uint16_t *lo, size_t M, size_t K, uint16_t *hi2,
-                        uint16_t *lo2, hipStream_t s);
-void launch_dequant(Dt wt, const void *values, const float *scales, size_t n, float *out,
-                    hipStream_t s);
 // decoder/weight_format.rs:150-183 on the device: rows x cols f32 (cols a
 // multiple of 32) to packed values + block scales.
 void launch_quantize(Dt wt, const float *src, size_t rows, size_t cols, void *values,

@@ -181,7 +181,7 @@ __global__ void __launch_bounds__(256) gemm_f32_k(GemmArgs g, float *ws, int k_p
 // K in 16-key stages and 16-byte aligned rows; f32 activations and output
 bool gemm_f32_ok(Dt wt, const GemmArgs &a) {
     auto al16 = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
-    return wt == DT_F32 && !a.a_lo && !a.c_lo && !a.kdup && a.K >= FG_BK && a.K % FG_BK == 0 &&
+    return wt == DT_F32 && !a.a_lo && !a.c_lo && a.K >= FG_BK && a.K % FG_BK == 0 &&
            a.grp_w_stride % 4 == 0 && al16(a.a) && al16(a.w) && (!a.w2 || al16(a.w2));
 }
 

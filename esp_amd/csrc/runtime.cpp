@@ -803,47 +803,6 @@ static void *lo_plane(Dt act, const DevMem &b, int rows, int cols) {
     return act == DT_SPLIT ? (void *)((uint16_t *)b.p + (size_t)rows * cols) : nullptr;
 }
 
-// GEMM weight operand: packed projections are dequantized to f32 first
-// (into slot 0 or 1 of kv.deq, in stream order before the GEMM reading it)
-// and multiplied by the f32 GEMM.
-static const void *gemm_w(Kv &kv, int slot, Dt wt, const void *w, const float *ws, size_t N,
-                          size_t K) {
-    if (!dt_packed(wt)) return w;
-    DevMem &d = kv.deq[slot];
-    d.ensure(N * K * 4);
-    launch_dequant(wt, w, ws, N * K, d.as<float>(), kv.stream);
-    return d.p;
-}
-static Dt gemm_dt(Dt wt) { return dt_packed(wt) ? DT_F32 : wt; }
-// Layer GEMMs of packed models run on the matrix cores in doubled-K form:
-// weights dequantized to [N, 2K] bf16 rows [hi | lo] (kernel comment in
-// k_moe.hip), activations (split planes) widened to [hi | hi], [lo | 0].
-static const void *gemm_w_split(Kv &kv, int slot, Dt wt, const void *w, const float *ws, size_t N,
-                                size_t K) {
-    if (!dt_packed(wt)) return w;
-    DevMem &d = kv.deq[slot];
-    d.ensure(N * K * 4);
-    launch_dequant_split(wt, w, ws, N, K, d.as<uint16_t>(), kv.stream);
-    return d.p;
-}
-static Dt layer_gemm_dt(Dt wt) { return dt_packed(wt) ? DT_BF16 : wt; }
-static void widen_k(const Model &m, Kv &kv, GemmArgs &g) {
-    if (!dt_packed(m.wt)) return;
-    if (g.M >= 1024 && g.K % 32 == 0 && !g.grp_offs) {
-        // the streamed GEMM reads the planes twice itself and skips the
-        // zero lo half (GemmArgs::kdup): no widened copy, 3/4 of the MFMAs
-        g.kdup = g.K;
-        g.K = 2 * g.K;
-        return;
-    }
-    const size_t M = g.M, K = g.K;
-    kv.wide.ensure(M * K * 8);
-    uint16_t *hi2 = kv.wide.as<uint16_t>(), *lo2 = hi2 + M * 2 * K;
-    launch_widen_split((const uint16_t *)g.a, (const uint16_t *)g.a_lo, M, K, hi2, lo2, kv.stream);
-    g.a = hi2;
-    g.a_lo = lo2;
-    g.K = (int)(2 * K);
-}
 // element type of LoRA B rows (packed formats carry no LoRA)
 static Dt lora_dt(Dt wt) { return dt_packed(wt) ? DT_F32 : wt; }
 
@@ -1170,7 +1129,8 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             g.ws_bytes = kv.gemm_ws.bytes;
             g.a = kv.xn.p;
             g.a_lo = lo_plane(act, kv.xn, Mc, H);
-            g.w = gemm_w_split(kv, 0, m.wt, w.qkv, w.qkv_s, w.qkv_rows, H);
+            g.w = w.qkv;
+            g.w_scale = w.qkv_s;
             g.bias = w.qkv_bias;
             g.c = kv.qkv.p;
             g.M = Mc;
@@ -1180,8 +1140,7 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             if (rope_kv_fusable(lora_dt(m.wt), kv.dt, m.hd, m.nq, m.nkv, lora_any))
                 g.defer_splits = &qkv_splits;
             Prof p("gemm_qkv", s);
-            widen_k(m, kv, g);
-            launch_gemm(layer_gemm_dt(m.wt), GEMM_STORE, g, s);
+            launch_gemm(m.wt, GEMM_STORE, g, s);
         }
         pre_normed = false;
         {
@@ -1304,7 +1263,8 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             g.ws_bytes = kv.gemm_ws.bytes;
             g.a = kv.attn.p;
             g.a_lo = lo_plane(act, kv.attn, Mc, m.qw);
-            g.w = gemm_w_split(kv, 0, m.wt, w.o, w.o_s, H, m.qw);
+            g.w = w.o;
+            g.w_scale = w.o_s;
             g.bias = w.o_bias;
             g.c = kv.h.p;
             g.M = Mc;
@@ -1313,8 +1273,7 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             g.ldc = H;
             if (!w.moe && resid_norm_ok(H)) g.defer_splits = &o_splits;
             Prof p("gemm_o", s);
-            widen_k(m, kv, g);
-            launch_gemm(layer_gemm_dt(m.wt), GEMM_RESIDUAL, g, s);
+            launch_gemm(m.wt, GEMM_RESIDUAL, g, s);
         }
         // ---- MLP block (layer.rs:147-151)
         if (w.moe) {
@@ -1356,8 +1315,10 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             g.ws_bytes = kv.gemm_ws.bytes;
             g.a = kv.xn.p;
             g.a_lo = lo_plane(act, kv.xn, Mc, H);
-            g.w = gemm_w_split(kv, 0, m.wt, w.gate, w.gate_s, m.F, H);
-            g.w2 = gemm_w_split(kv, 1, m.wt, w.up, w.up_s, m.F, H);
+            g.w = w.gate;
+            g.w_scale = w.gate_s;
+            g.w2 = w.up;
+            g.w2_scale = w.up_s;
             g.c = kv.act.p;
             g.c_lo = lo_plane(act, kv.act, Mc, m.F);
             g.M = Mc;
@@ -1366,15 +1327,15 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             g.ldc = m.F;
             {
                 Prof p("gemm_mlp", s);
-                widen_k(m, kv, g);
-                launch_gemm(layer_gemm_dt(m.wt), GEMM_SWIGLU, g, s);
+                launch_gemm(m.wt, GEMM_SWIGLU, g, s);
             }
             GemmArgs d{};
             d.ws = kv.gemm_ws.as<float>();
             d.ws_bytes = kv.gemm_ws.bytes;
             d.a = kv.act.p;
             d.a_lo = lo_plane(act, kv.act, Mc, m.F);
-            d.w = gemm_w_split(kv, 0, m.wt, w.down, w.down_s, H, m.F);
+            d.w = w.down;
+            d.w_scale = w.down_s;
             d.c = kv.h.p;
             d.M = Mc;
             d.N = H;
@@ -1386,8 +1347,7 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             if (next_norm) d.defer_splits = &d_splits;
             {
                 Prof p("gemm_down", s);
-                widen_k(m, kv, d);
-                launch_gemm(layer_gemm_dt(m.wt), GEMM_RESIDUAL, d, s);
+                launch_gemm(m.wt, GEMM_RESIDUAL, d, s);
             }
             if (d_splits > 1) {
                 Prof p("resid_norm", s);
@@ -1506,24 +1466,25 @@ static void run_head(Model &m, Kv &kv, int n_seqs, const float *h_src, const int
         launch_gemv(m.ht, GEMV_STORE, g, s);
         return;
     }
+    const Dt act = m.ht == DT_F32 ? DT_F32 : DT_SPLIT;
     {
         Prof p("rmsnorm", s);
-        launch_rmsnorm(h_src, m.final_norm, m.cfg.rms_norm_eps, n_seqs, m.H,
-                       m.ht == DT_BF16 ? DT_SPLIT : DT_F32, kv.xn.p, row_index, s);
+        launch_rmsnorm(h_src, m.final_norm, m.cfg.rms_norm_eps, n_seqs, m.H, act, kv.xn.p, row_index, s);
     }
     GemmArgs g{};
     g.ws = kv.gemm_ws.as<float>();
     g.ws_bytes = kv.gemm_ws.bytes;
     g.a = kv.xn.p;
-    g.a_lo = lo_plane(m.ht == DT_BF16 ? DT_SPLIT : DT_F32, kv.xn, n_seqs, m.H);
-    g.w = gemm_w(kv, 0, m.ht, m.head, m.head_s, m.V, m.H);
+    g.a_lo = lo_plane(act, kv.xn, n_seqs, m.H);
+    g.w = m.head;
+    g.w_scale = m.head_s;
     g.c = kv.logits.p;
     g.M = n_seqs;
     g.N = m.V;
     g.K = m.H;
     g.ldc = m.V;
     Prof p("gemm", s);
-    launch_gemm(gemm_dt(m.ht), GEMM_STORE, g, s);
+    launch_gemm(m.ht, GEMM_STORE, g, s);
 }
 
 // After a stream has drained: whether a decode-attention launch since the

@@ -106,8 +106,6 @@ struct Kv {
     DevMem rows_dev;   // ids | row_seq | row_pos | last_row  (int32)
     DevMem h, xn, qkv, q, attn, act, part, last_h, logits, pick_scratch, pick_io;
     DevMem gemm_ws;  // split-K partial sums of the prefill GEMMs
-    DevMem deq[2];   // packed formats: dequantized weights of the GEMMs in flight
-    DevMem wide;     // packed formats: activation planes widened to the doubled K
     DevMem tickets;  // zeroed counters for last-block merges (attention, head argmax)
     // the decode position's rope rows (cos then sin, hd floats each), written
     // by the single-row QKV launch for the attention's LoRA deltas

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from esp_amd import DecoderModel
-from oracle import oracle, st
+from oracle import oracle, quant, st
 from tests import synth
 
 pytestmark = pytest.mark.gpu
@@ -36,3 +36,20 @@ def test_f32_rows(hidden, ffn, rows):
     cfg, tensors, blob, _ = synth.tiny_llama_case(seed=5, layers=2, hidden=hidden, heads=hidden // 16,
                                                   kv_heads=hidden // 16, ffn=ffn, vocab=131, prompt_len=2)
     _rows_match(DecoderModel.from_bytes(cfg, blob, "f32"), oracle.OracleModel(cfg, tensors), 131, rows, 1e-4)
+
+
+# K 96 (no skinny form: K % 128), 256 (skinny at both row counts), 640 =
+# K % 128 only, and k splits with a ragged last one at 1408
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("hidden,ffn", [(128, 192), (256, 640), (512, 1408)])
+@pytest.mark.parametrize("rows", [2, 31, 32, 33, 64, 65, 129, 300])
+def test_packed_rows(bits, hidden, ffn, rows):
+    """Packed projections and head over several rows: 1e-4 of the row's
+    magnitude (activations as two bf16 halves, 2^-17 a product)."""
+    print(f"q{bits} rows {rows} hidden {hidden} ffn {ffn}", flush=True)
+    cfg = synth.llama_config(2, hidden, 4, 2, ffn, 131, head_dim=32 if hidden < 512 else 64)
+    tensors = synth.make_tensors(cfg, 9, "f32", std=0.05)
+    art = quant.convert_artifact(tensors, bits)
+    shapes = {n: a.shape for n, (a, _) in tensors.items()}
+    ref = oracle.OracleModel(cfg, quant.dequantized_model(art, shapes, bits))
+    _rows_match(DecoderModel.from_bytes(cfg, st.dump(art), f"q{bits}-block32"), ref, 131, rows, 1e-4)
