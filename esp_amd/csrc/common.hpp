@@ -75,6 +75,12 @@ void launch_resid_norm(const float *ws, int splits, int M, int H, const float *b
 void launch_rmsnorm(const float *x, const float *gamma, float eps, int M, int H, Dt out_dt,
                     void *out, const int32_t *row_index, hipStream_t s);
 
+// h[m] = embed[ids[m]] and out[m] = RMSNorm(h[m]) * gamma (DT_SPLIT planes or
+// f32), where embed_norm_ok.
+bool embed_norm_ok(Dt wt, const void *embed, int H);
+void launch_embed_norm(Dt wt, const void *embed, const int32_t *ids, int M, int H, float *h,
+                       const float *gamma, float eps, Dt out_dt, void *out, hipStream_t s);
+
 // GEMV (one input row): y = W x with the input RMS-normalised on the fly
 // when gamma != nullptr. Epilogue kinds below.
 enum GemvEpi { GEMV_STORE = 0, GEMV_RESIDUAL = 1, GEMV_SWIGLU = 2 };

@@ -17,12 +17,37 @@ __global__ void __launch_bounds__(256) embed_k(const WT *E, const int32_t *ids, 
     for (int j = threadIdx.x; j < H; j += blockDim.x) h[(size_t)m * H + j] = ld(row, j);
 }
 
+// four elements of an embedding row
+__device__ __forceinline__ f32x4 ld4(const float *p) { return *(const f32x4 *)p; }
+__device__ __forceinline__ f32x4 ld4(const uint16_t *p) {
+    const uint2 u = *(const uint2 *)p;
+    return f32x4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                 __uint_as_float(u.y & 0xffff0000u)};
+}
+
+// Four elements per thread (H % 4 == 0, aligned rows), every load in one
+// round trip: one element per thread and iteration waited for each of 16
+// trips at H 4096 (one row of bf16 4.4 -> 3.4 us).
+template <typename WT>
+__global__ void __launch_bounds__(256) embed4_k(const WT *E, const int32_t *ids, int H, float *h) {
+    const int m = blockIdx.x, j = (blockIdx.y * 256 + threadIdx.x) * 4;
+    if (j < H) *(f32x4 *)(h + (size_t)m * H + j) = ld4(E + (size_t)ids[m] * H + j);
+}
+
+static bool aligned(const void *p, size_t n) { return (uintptr_t)p % n == 0; }
+
+template <typename WT>
+static void embed_launch(const WT *E, const int32_t *ids, int M, int H, float *h, hipStream_t s) {
+    if (H % 4 == 0 && aligned(E, 4 * sizeof(WT)) && aligned(h, 16))
+        embed4_k<WT><<<dim3(M, (H / 4 + 255) / 256), 256, 0, s>>>(E, ids, H, h);
+    else
+        embed_k<WT><<<M, 256, 0, s>>>(E, ids, H, h);
+}
+
 void launch_embed(Dt wt, const void *embed, const int32_t *ids, int M, int H, float *h,
                   hipStream_t s) {
-    if (wt == DT_BF16)
-        embed_k<uint16_t><<<M, 256, 0, s>>>((const uint16_t *)embed, ids, H, h);
-    else
-        embed_k<float><<<M, 256, 0, s>>>((const float *)embed, ids, H, h);
+    if (wt == DT_BF16) embed_launch((const uint16_t *)embed, ids, M, H, h, s);
+    else embed_launch((const float *)embed, ids, M, H, h, s);
 }
 
 // ---------------------------------------------------------------- rmsnorm
@@ -46,78 +71,140 @@ __global__ void __launch_bounds__(256) rmsnorm_k(const float *x, const float *ga
     }
 }
 
-// One wave per row for rows up to 4096 wide: the row and the norm weights
-// stay in registers (NQ four-element pieces per lane, 16-byte loads issued
-// together), the sum of squares is a wave reduction, and the output goes out
-// four elements per store.
-template <typename OT, bool SPLIT, int NQ>
-__global__ void __launch_bounds__(256) rmsnorm_wave_k(const float *x, const float *gamma, float eps, int M,
-                                                      int H, OT *out, const int32_t *row_index) {
-    const int lane = threadIdx.x & 63;
-    const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (m >= M) return;
-    const int src = row_index ? row_index[m] : m;
-    const float *xr = x + (size_t)src * H;
-    f32x4 v[NQ], gv[NQ];  // the row and the norm weights, loaded together
-    float ss = 0.f;
+// One block per row, four elements per thread (eight above H 4096), so the
+// row, the norm weights and what feeds the row arrive in one round trip; a
+// few rows are bound by that trip and the block's two meetings, many rows by
+// memory. Three sources of the row:
+//   NB_PLAIN  x[row_index ? row_index[m] : m]
+//   NB_RESID  x[m] += bias + the split-K partial sums of a RESIDUAL
+//             projection (layer.rs:120-151: o_proj before the post-attention
+//             norm, down_proj before the next layer's input norm), summed
+//             from 0 in split order, eight loads in flight, as the GEMM
+//             reduction does
+//   NB_EMBED  x[m] = embedding row ids[m], the first layer's input
+// Measured at H 4096, four rows: plain 12.8 -> 4.7 us (was one wave per row),
+// resid 9.2 -> 5.6 us (was 256 threads, a trip per quarter row), embedding and
+// norm 23.4 -> 6.3 us; 2048 rows: resid 32.6 -> 31.7, embedding and norm 43.5
+// -> 26.9 us.
+enum { NB_PLAIN = 0, NB_RESID = 1, NB_EMBED = 2 };
+struct NormArgs {
+    float *x;                  // [M, H] residual stream
+    const float *gamma;
+    float eps;
+    int M, H;
+    void *out;                 // f32 [M, H], or hi / lo planes of M rows
+    const int32_t *row_index;  // PLAIN: nullable
+    const float *ws, *bias;    // RESID: [splits][M][H], nullable [H]
+    int splits;
+    const void *embed;         // EMBED: [V, H]
+    const int32_t *ids;
+};
+
+template <bool SPLIT, int NT, int NQ, int MODE, typename ET>
+__global__ void __launch_bounds__(NT) norm_block_k(NormArgs a) {
+    __shared__ float sq[NT * NQ];
+    const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, H = a.H;
+    const size_t MH = (size_t)a.M * H;
+    const size_t src = MODE == NB_PLAIN && a.row_index ? (size_t)a.row_index[m] * H : (size_t)m * H;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v[NQ], gv[NQ];
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
-        const int j = (lane + 64 * i) * 4;
-        v[i] = j < H ? *(const f32x4 *)(xr + j) : f32x4{0.f, 0.f, 0.f, 0.f};
-        gv[i] = j < H ? *(const f32x4 *)(gamma + j) : f32x4{0.f, 0.f, 0.f, 0.f};
+        const int j = (tid + NT * i) * 4;
+        v[i] = gv[i] = zero;
+        if (j >= H) continue;
+        gv[i] = *(const f32x4 *)(a.gamma + j);
+        if (MODE == NB_EMBED) {
+            v[i] = ld4((const ET *)a.embed + (size_t)a.ids[m] * H + j);
+            *(f32x4 *)(a.x + src + j) = v[i];
+            continue;
+        }
+        v[i] = *(const f32x4 *)(a.x + src + j);
+        if (MODE == NB_RESID) {
+            const float *w = a.ws + src + j;
+            f32x4 t = zero;
+            for (int z0 = 0; z0 < a.splits; z0 += 8) {
+                f32x4 pz[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    pz[q] = z0 + q < a.splits ? *(const f32x4 *)(w + (size_t)(z0 + q) * MH) : zero;
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    if (z0 + q < a.splits) t += pz[q];
+            }
+            if (a.bias) t = t + *(const f32x4 *)(a.bias + j);
+            v[i] = v[i] + t;
+            *(f32x4 *)(a.x + src + j) = v[i];
+        }
     }
+    // The sum of squares in an order that does not depend on the block's
+    // size: every wave adds the quads' sums itself, PLAIN and EMBED as lane l
+    // over quads l + 64 i, RESID as four parts over quads 64 p + l + 256 i.
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) ss += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
-    ss = wave_sum(ss);
-    const float rms = sqrtf(ss / (float)H + eps);
-    const size_t plane = (size_t)M * H;
+    for (int i = 0; i < NQ; ++i)
+        sq[tid + NT * i] = v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
+    __syncthreads();
+    constexpr int NP = MODE == NB_RESID && NT >= 128 ? (NT >= 256 ? 4 : 2) : 1;
+    float part[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+#pragma unroll
+        for (int i = 0; i < NT * NQ / (64 * NP); ++i) part[p] += sq[64 * p + lane + 64 * NP * i];
+        part[p] = wave_sum(part[p]);
+    }
+    const float ss = (part[0] + part[1]) + (part[2] + part[3]);
+    const float rms = sqrtf(ss / (float)H + a.eps);
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
-        const int j = (lane + 64 * i) * 4;
+        const int j = (tid + NT * i) * 4;
         if (j >= H) continue;
         float y[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = (v[i][e] / rms) * gv[i][e];
         const size_t o = (size_t)m * H + j;
         if (SPLIT) {
+            uint16_t *out = (uint16_t *)a.out;
             uint16_t hi[4], lo[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 hi[e] = f2bf(y[e]);
                 lo[e] = f2bf(y[e] - bf2f(hi[e]));
             }
-            *(uint2 *)((uint16_t *)out + o) = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
-            *(uint2 *)((uint16_t *)out + plane + o) =
-                make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
-        } else if (sizeof(OT) == 2) {
-            uint16_t b[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) b[e] = f2bf(y[e]);
-            *(uint2 *)((uint16_t *)out + o) = make_uint2(b[0] | ((uint32_t)b[1] << 16), b[2] | ((uint32_t)b[3] << 16));
+            *(uint2 *)(out + o) = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
+            *(uint2 *)(out + MH + o) = make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
         } else {
-            *(f32x4 *)((float *)out + o) = f32x4{y[0], y[1], y[2], y[3]};
+            *(f32x4 *)((float *)a.out + o) = f32x4{y[0], y[1], y[2], y[3]};
         }
     }
 }
 
-template <typename OT, bool SPLIT>
-static bool rmsnorm_wave(const float *x, const float *gamma, float eps, int M, int H, OT *out,
-                         const int32_t *row_index, hipStream_t s) {
-    if (H % 4 || H > 4096) return false;
-    const int nq = (H / 4 + 63) / 64;
-    const int blocks = (M + 3) / 4;
-    if (nq <= 2) rmsnorm_wave_k<OT, SPLIT, 2><<<blocks, 256, 0, s>>>(x, gamma, eps, M, H, out, row_index);
-    else if (nq <= 4) rmsnorm_wave_k<OT, SPLIT, 4><<<blocks, 256, 0, s>>>(x, gamma, eps, M, H, out, row_index);
-    else if (nq <= 8) rmsnorm_wave_k<OT, SPLIT, 8><<<blocks, 256, 0, s>>>(x, gamma, eps, M, H, out, row_index);
-    else rmsnorm_wave_k<OT, SPLIT, 16><<<blocks, 256, 0, s>>>(x, gamma, eps, M, H, out, row_index);
-    return true;
+template <bool SPLIT, int MODE, typename ET> static void norm_block(const NormArgs &a, hipStream_t s) {
+    const int q = a.H / 4;
+    if (q <= 64) norm_block_k<SPLIT, 64, 1, MODE, ET><<<a.M, 64, 0, s>>>(a);
+    else if (q <= 128) norm_block_k<SPLIT, 128, 1, MODE, ET><<<a.M, 128, 0, s>>>(a);
+    else if (q <= 256) norm_block_k<SPLIT, 256, 1, MODE, ET><<<a.M, 256, 0, s>>>(a);
+    else if (q <= 512) norm_block_k<SPLIT, 512, 1, MODE, ET><<<a.M, 512, 0, s>>>(a);
+    else if (q <= 1024) norm_block_k<SPLIT, 1024, 1, MODE, ET><<<a.M, 1024, 0, s>>>(a);
+    else norm_block_k<SPLIT, 1024, 2, MODE, ET><<<a.M, 1024, 0, s>>>(a);
 }
+
+bool resid_norm_ok(int H) { return H > 0 && H % 4 == 0 && H <= 8192; }
 
 void launch_rmsnorm(const float *x, const float *gamma, float eps, int M, int H, Dt out_dt,
                     void *out, const int32_t *row_index, hipStream_t s) {
-    if (out_dt == DT_SPLIT && rmsnorm_wave<uint16_t, true>(x, gamma, eps, M, H, (uint16_t *)out, row_index, s)) return;
-    if (out_dt == DT_BF16 && rmsnorm_wave<uint16_t, false>(x, gamma, eps, M, H, (uint16_t *)out, row_index, s)) return;
-    if (out_dt == DT_F32 && rmsnorm_wave<float, false>(x, gamma, eps, M, H, (float *)out, row_index, s)) return;
+    if (resid_norm_ok(H) && out_dt != DT_BF16) {
+        NormArgs a{};
+        a.x = const_cast<float *>(x);  // read only in this mode
+        a.gamma = gamma;
+        a.eps = eps;
+        a.M = M;
+        a.H = H;
+        a.out = out;
+        a.row_index = row_index;
+        if (out_dt == DT_SPLIT) norm_block<true, NB_PLAIN, float>(a, s);
+        else norm_block<false, NB_PLAIN, float>(a, s);
+        return;
+    }
     if (out_dt == DT_SPLIT)
         rmsnorm_k<uint16_t, true><<<M, 256, 0, s>>>(x, gamma, eps, H, (uint16_t *)out, row_index);
     else if (out_dt == DT_BF16)
@@ -126,96 +213,43 @@ void launch_rmsnorm(const float *x, const float *gamma, float eps, int M, int H,
         rmsnorm_k<float, false><<<M, 256, 0, s>>>(x, gamma, eps, H, (float *)out, row_index);
 }
 
-// Split-K partial sums of a RESIDUAL projection fused with the RMSNorm that
-// follows it (layer.rs:120-151: the o_proj residual before post-attention
-// norm, the down_proj residual before the next layer's input norm). One
-// block per row; thread t owns elements 4 (t + 256 i) .. + 4. The partials
-// are summed from 0 in split order, eight loads in flight, then + bias and
-// added to x, exactly as the GEMM reduction does; the norm is then that of
-// rmsnorm_k on the new row.
-template <typename OT, bool SPLIT, int NQ>
-__global__ void __launch_bounds__(256) resid_norm_k(const float *ws, int splits, int M, int H,
-                                                    const float *bias, float *x, const float *gamma,
-                                                    float eps, OT *out) {
-    __shared__ float red[4];
-    const int m = blockIdx.x, tid = threadIdx.x;
-    const size_t MH = (size_t)M * H;
-    f32x4 v[NQ], gv[NQ];
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-        const int j = (tid + 256 * i) * 4;
-        v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (j >= H) continue;
-        // gamma now, with the partials: no memory wait after the barrier
-        gv[i] = *(const f32x4 *)(gamma + j);
-        const size_t o = (size_t)m * H + j;
-        f32x4 t = {0.f, 0.f, 0.f, 0.f};
-        for (int z0 = 0; z0 < splits; z0 += 8) {
-            f32x4 pz[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-                pz[q] = z0 + q < splits ? *(const f32x4 *)(ws + (size_t)(z0 + q) * MH + o) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-                if (z0 + q < splits) t += pz[q];
-        }
-        if (bias) t = t + *(const f32x4 *)(bias + j);
-        const f32x4 xv = *(const f32x4 *)(x + o) + t;
-        *(f32x4 *)(x + o) = xv;
-        v[i] = xv;
-        ss += xv[0] * xv[0] + xv[1] * xv[1] + xv[2] * xv[2] + xv[3] * xv[3];
-    }
-    ss = wave_sum(ss);
-    if ((tid & 63) == 0) red[tid >> 6] = ss;
-    __syncthreads();
-    ss = (red[0] + red[1]) + (red[2] + red[3]);
-    const float rms = sqrtf(ss / (float)H + eps);
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-        const int j = (tid + 256 * i) * 4;
-        if (j >= H) continue;
-        float y[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = (v[i][e] / rms) * gv[i][e];
-        const size_t o = (size_t)m * H + j;
-        if (SPLIT) {
-            uint16_t hi[4], lo[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                hi[e] = f2bf(y[e]);
-                lo[e] = f2bf(y[e] - bf2f(hi[e]));
-            }
-            *(uint2 *)((uint16_t *)out + o) = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
-            *(uint2 *)((uint16_t *)out + MH + o) =
-                make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
-        } else {
-            *(f32x4 *)((float *)out + o) = f32x4{y[0], y[1], y[2], y[3]};
-        }
-    }
-}
-
-bool resid_norm_ok(int H) { return H > 0 && H % 4 == 0 && H <= 8192; }
-
 void launch_resid_norm(const float *ws, int splits, int M, int H, const float *bias, float *x,
                        const float *gamma, float eps, Dt out_dt, void *out, hipStream_t s) {
     if (!resid_norm_ok(H) || splits < 1 || (out_dt != DT_SPLIT && out_dt != DT_F32))
         fail(ESP_BACKEND, "resid_norm: unsupported shape");
-    const int nq = (H / 4 + 255) / 256;
-#define RN_LAUNCH(NQ_)                                                                                    \
-    do {                                                                                                  \
-        if (out_dt == DT_SPLIT)                                                                           \
-            resid_norm_k<uint16_t, true, NQ_><<<M, 256, 0, s>>>(ws, splits, M, H, bias, x, gamma, eps,    \
-                                                                 (uint16_t *)out);                        \
-        else                                                                                              \
-            resid_norm_k<float, false, NQ_><<<M, 256, 0, s>>>(ws, splits, M, H, bias, x, gamma, eps,      \
-                                                               (float *)out);                             \
-    } while (0)
-    if (nq <= 1) RN_LAUNCH(1);
-    else if (nq <= 2) RN_LAUNCH(2);
-    else if (nq <= 4) RN_LAUNCH(4);
-    else RN_LAUNCH(8);
-#undef RN_LAUNCH
+    NormArgs a{};
+    a.x = x;
+    a.gamma = gamma;
+    a.eps = eps;
+    a.M = M;
+    a.H = H;
+    a.out = out;
+    a.ws = ws;
+    a.bias = bias;
+    a.splits = splits;
+    if (out_dt == DT_SPLIT) norm_block<true, NB_RESID, float>(a, s);
+    else norm_block<false, NB_RESID, float>(a, s);
+}
+
+bool embed_norm_ok(Dt wt, const void *embed, int H) {
+    return resid_norm_ok(H) && aligned(embed, wt == DT_BF16 ? 8 : 16);
+}
+
+void launch_embed_norm(Dt wt, const void *embed, const int32_t *ids, int M, int H, float *h,
+                       const float *gamma, float eps, Dt out_dt, void *out, hipStream_t s) {
+    NormArgs a{};
+    a.x = h;
+    a.gamma = gamma;
+    a.eps = eps;
+    a.M = M;
+    a.H = H;
+    a.out = out;
+    a.embed = embed;
+    a.ids = ids;
+    if (wt == DT_BF16 && out_dt == DT_SPLIT) norm_block<true, NB_EMBED, uint16_t>(a, s);
+    else if (wt == DT_BF16) norm_block<false, NB_EMBED, uint16_t>(a, s);
+    else if (out_dt == DT_SPLIT) norm_block<true, NB_EMBED, float>(a, s);
+    else norm_block<false, NB_EMBED, float>(a, s);
 }
 
 // ----------------------------------------------------------------- rope_kv

@@ -1065,13 +1065,30 @@ struct Seg {
     int seq, row0, len, p0;
 };
 
+// The activation kind that `m`'s projections of several rows read: bf16 and
+// packed weights take split hi/lo bf16 planes to the matrix cores, f32 models
+// plain f32.
+static Dt act_dt(const Model &m) { return m.wt == DT_BF16 || dt_packed(m.wt) ? DT_SPLIT : DT_F32; }
+
+// kv.h = the token rows' embeddings and, for several rows into a resident
+// first layer, kv.xn = their input RMSNorm; returns whether it did the norm.
+static bool embed_rows(Model &m, Kv &kv, const int32_t *ids, int Mc) {
+    Prof p("embed", kv.stream);
+    if (Mc > 1 && !m.st && embed_norm_ok(m.et, m.embed, m.H)) {
+        launch_embed_norm(m.et, m.embed, ids, Mc, m.H, kv.h.as<float>(), m.layers[0].in_norm,
+                          m.cfg.rms_norm_eps, act_dt(m), kv.xn.p, kv.stream);
+        return true;
+    }
+    launch_embed(m.et, m.embed, ids, Mc, m.H, kv.h.as<float>(), kv.stream);
+    return false;
+}
+
+// `pre_normed`: kv.xn already holds the first layer's input norm.
 static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, int one_seq = -1,
-                       int p0 = 0, const std::vector<Seg> *segs = nullptr) {
+                       int p0 = 0, const std::vector<Seg> *segs = nullptr, bool pre_normed = false) {
     hipStream_t s = kv.stream;
     const bool single = Mc == 1;
-    // activations keep f32 precision; bf16 models hand them to the matrix
-    // cores as split hi/lo bf16 planes, f32 models as plain f32
-    const Dt act = m.wt == DT_BF16 || dt_packed(m.wt) ? DT_SPLIT : DT_F32;
+    const Dt act = act_dt(m);
     const int H = m.H;
     const bool dec_attn = use_attn_decode(m, kv, Mc);
     Plan plan = attn_plan(m, Mc, max_t);
@@ -1092,7 +1109,6 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
     // the rotary/KV kernel, the o_proj and down_proj residual sums by a row
     // kernel that also applies the next RMSNorm (post-attention, or the next
     // resident layer's input norm: `pre_normed`).
-    bool pre_normed = false;
     for (int l = 0; l < m.L; ++l) {
         LayerW staged;
         if (m.st) staged = stream_acquire(m, kv, l);
@@ -1596,12 +1612,9 @@ static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, con
             rows.ngrp = ngrp;
             rows.grp_rows = grp_rows;
         }
-        {
-            Prof p("embed", s);
-            launch_embed(m.et, m.embed, rows.ids, Mc, m.H, kv.h.as<float>(), s);
-        }
-        if (n_seqs == 1) run_layers(m, kv, rows, Mc, max_t, (int)seqs[0], rpos[c0]);
-        else run_layers(m, kv, rows, Mc, max_t, -1, 0, &segs);
+        const bool normed = embed_rows(m, kv, rows.ids, Mc);
+        if (n_seqs == 1) run_layers(m, kv, rows, Mc, max_t, (int)seqs[0], rpos[c0], nullptr, normed);
+        else run_layers(m, kv, rows, Mc, max_t, -1, 0, &segs, normed);
         if (one_chunk) break;
         // keep the hidden state of every sequence's last row in this chunk
         for (int i = 0; i < n_seqs; ++i)
@@ -1704,10 +1717,7 @@ void decode_step_dev(Model &m, Kv &kv, int seq, int max_t, int32_t *gen) {
         ~StepWord() { k.gen_step = nullptr; }
     } step_word(kv, gen + 1);
     Rows rows{gen, gen + 2, gen + 3, 1, seq};
-    {
-        Prof p("embed", s);
-        launch_embed(m.et, m.embed, rows.ids, 1, m.H, kv.h.as<float>(), s);
-    }
+    embed_rows(m, kv, rows.ids, 1);
     run_layers(m, kv, rows, 1, max_t);
     if (decode_gemv_ok(m.H)) {
         run_head(m, kv, 1, kv.h.as<float>(), nullptr, gen);  // argmax + hand-off fused
