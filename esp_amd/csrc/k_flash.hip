@@ -430,13 +430,31 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     // Work: a group is (pair of query blocks, kv head); its G query heads run
     // on one XCD (workgroups are dealt to the XCDs round-robin by linear id)
     // so they share K/V tiles in that XCD's L2.
-    const int npair = (nqb + 1) / 2;
-    const int G = a.nq / a.nkv, ngroups = npair * a.nkv;
+    // Several sequences' prompt blocks share a launch (a launch each left most
+    // of the chip idle: twelve blocks of 24-283 rows, hd 64, f16 cache, 179 ->
+    // 34 us per layer).
+    const int G = a.nq / a.nkv, ngroups = (a.units ? a.n_units : (nqb + 1) / 2) * a.nkv;
     const int xcd = blockIdx.x % FA_XCDS, slot = blockIdx.x / FA_XCDS;
     const int gi = (slot / G) * FA_XCDS + xcd;
     if (gi >= ngroups) return;
-    const int pr = gi / a.nkv, kvh = gi % a.nkv;
-    const int qh = kvh * G + slot % G;
+    int pr = gi / a.nkv;
+    const int kvh = gi % a.nkv, qh = kvh * G + slot % G;
+    if (a.units) {
+        const FlashUnit u = a.units[pr];
+        const size_t off = (size_t)u.row0 * a.nq * HD;
+        a.q += off;
+        if (a.out_lo) {
+            a.out = (float *)((uint16_t *)a.out + off);  // the hi plane's bf16 rows
+            a.out_lo += off;
+        } else {
+            a.out += off;
+        }
+        a.M = u.len;
+        a.seq = u.seq;
+        a.p0 = u.p0;
+        pr = u.pr;
+        nqb = u.nqb;
+    }
     flash_block<HD, F16>(a, nqb - 1 - pr, qh, kvh, fl);
     if (pr != nqb - 1 - pr) {
         __syncthreads();  // the first block's merge rows are read
@@ -457,10 +475,10 @@ template <int HD, bool F16> static void flash_launch(const FlashArgs &a, int nqb
 }
 
 void launch_flash(const FlashArgs &a, hipStream_t s) {
-    if (a.M <= 0) return;
+    if (a.units ? a.n_units <= 0 : a.M <= 0) return;
     if (a.nkv <= 0 || a.nq % a.nkv != 0) fail(ESP_BACKEND, "flash attention: bad head grouping");
     const int nqb = (a.M + FA_BQ - 1) / FA_BQ;
-    const int G = a.nq / a.nkv, ngroups = (nqb + 1) / 2 * a.nkv;
+    const int G = a.nq / a.nkv, ngroups = (a.units ? a.n_units : (nqb + 1) / 2) * a.nkv;
     const int blocks = ((ngroups + FA_XCDS - 1) / FA_XCDS) * FA_XCDS * G;
     if (a.hd == 64) {
         if (a.kv_f16) flash_launch<64, true>(a, nqb, blocks, s);

@@ -762,7 +762,7 @@ static void *kv_layer(Kv &kv, int l) {
     return (char *)kv.cache.p + (size_t)l * kv.layer_stride * dt_size(kv.dt);
 }
 
-static const int kMaxRows = 4096;  // token rows per pass through the layers
+static constexpr int kMaxRows = 4096;  // token rows per pass through the layers
 
 static void ensure_pinned(Kv &kv, size_t bytes) {
     if (kv.pinned_bytes >= bytes) return;
@@ -1065,6 +1065,35 @@ struct Seg {
     int seq, row0, len, p0;
 };
 
+// The flash attention's units of a chunk whose segments all have 16 rows or
+// more (n 0: some have fewer, or one sequence only).
+struct FlashUnits {
+    const FlashUnit *dev = nullptr;
+    int n = 0;
+};
+constexpr int kMinFlashSeg = 16;
+// a segment of len >= 16 rows has at most 1 + len / 256 pairs
+constexpr int kMaxFlashUnits = kMaxRows / kMinFlashSeg + kMaxRows / 256;
+constexpr int kUnitWords = sizeof(FlashUnit) / 4;
+
+// Writes the units of `segs` (longest key range first, so that the last ones
+// to start are short) to `out`; 0 if a segment is shorter than 16 rows.
+static int flash_units(const std::vector<Seg> &segs, FlashUnit *out) {
+    int n = 0;
+    for (const Seg &g : segs) {
+        if (g.len < kMinFlashSeg) return 0;
+        const int nqb = (g.len + 127) / 128;
+        for (int pr = 0; pr < (nqb + 1) / 2; ++pr) out[n++] = FlashUnit{g.row0, g.len, g.seq, g.p0, pr, nqb, {0, 0}};
+    }
+    auto keys = [](const FlashUnit &u) {  // of both blocks
+        const int hi = u.nqb - 1 - u.pr;
+        const int a = std::min(u.len, (hi + 1) * 128) + u.p0, b = (u.pr + 1) * 128 + u.p0;
+        return hi == u.pr ? a : a + b;
+    };
+    std::stable_sort(out, out + n, [&](const FlashUnit &x, const FlashUnit &y) { return keys(x) > keys(y); });
+    return n;
+}
+
 // The activation kind that `m`'s projections of several rows read: bf16 and
 // packed weights take split hi/lo bf16 planes to the matrix cores, f32 models
 // plain f32.
@@ -1085,7 +1114,7 @@ static bool embed_rows(Model &m, Kv &kv, const int32_t *ids, int Mc) {
 
 // `pre_normed`: kv.xn already holds the first layer's input norm.
 static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, int one_seq = -1,
-                       int p0 = 0, const std::vector<Seg> *segs = nullptr, bool pre_normed = false) {
+                       int p0 = 0, const FlashUnits &units = {}, bool pre_normed = false) {
     hipStream_t s = kv.stream;
     const bool single = Mc == 1;
     const Dt act = act_dt(m);
@@ -1192,33 +1221,25 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             Prof p("rope_kv", s);
             launch_rope_kv(lora_dt(m.wt), kv.dt, r, s);
         }
-        bool seg_flash = segs && !segs->empty() && act == DT_SPLIT && flash_ok(m.hd);
-        for (size_t i = 0; seg_flash && i < segs->size(); ++i) seg_flash = (*segs)[i].len >= 16;
-        if (seg_flash) {
-            // several sequences' prompt blocks: the tiled MFMA attention per block
-            uint16_t *lo = (uint16_t *)lo_plane(act, kv.attn, Mc, m.qw);
+        if (units.n && act == DT_SPLIT && flash_ok(m.hd)) {
+            // several sequences' prompt blocks: the tiled MFMA attention, one launch
+            FlashArgs f{};
+            f.q = kv.q.as<float>();
+            f.kv = kv_layer(kv, l);
+            f.kv_f16 = kv.dt == DT_F16;
+            f.seq_stride = kv.seq_stride;
+            f.kv_half_stride = kv.half_stride;
+            f.head_stride = kv.head_stride;
+            f.nq = m.nq;
+            f.nkv = m.nkv;
+            f.hd = m.hd;
+            f.window = w.window;
+            f.out = kv.attn.as<float>();
+            f.out_lo = (uint16_t *)lo_plane(act, kv.attn, Mc, m.qw);
+            f.units = units.dev;
+            f.n_units = units.n;
             Prof p("attention", s);
-            for (const Seg &g : *segs) {
-                FlashArgs f{};
-                f.q = kv.q.as<float>() + (size_t)g.row0 * m.qw;
-                f.kv = kv_layer(kv, l);
-                f.kv_f16 = kv.dt == DT_F16;
-                f.seq_stride = kv.seq_stride;
-                f.kv_half_stride = kv.half_stride;
-                f.head_stride = kv.head_stride;
-                f.seq = g.seq;
-                f.p0 = g.p0;
-                f.M = g.len;
-                f.nq = m.nq;
-                f.nkv = m.nkv;
-                f.hd = m.hd;
-                f.window = w.window;
-                // f32 rows, or the hi plane's bf16 rows when split
-                f.out = lo ? (float *)(kv.attn.as<uint16_t>() + (size_t)g.row0 * m.qw)
-                           : kv.attn.as<float>() + (size_t)g.row0 * m.qw;
-                f.out_lo = lo ? lo + (size_t)g.row0 * m.qw : nullptr;
-                launch_flash(f, s);
-            }
+            launch_flash(f, s);
         } else if (one_seq >= 0 && Mc >= 16 && act == DT_SPLIT && flash_ok(m.hd)) {
             // rows are consecutive positions of one sequence: tiled MFMA attention
             FlashArgs f{};
@@ -1389,7 +1410,7 @@ static void ensure_scratch(Model &m, Kv &kv, int Mc, int n_seqs) {
     kv.act.ensure((size_t)Mc * fmax * 4);
     kv.last_h.ensure((size_t)n_seqs * H * 4);
     kv.logits.ensure((size_t)std::max(n_seqs, kv.batch) * m.V * 4);
-    kv.rows_dev.ensure((size_t)(4 * kMaxRows + 2 * kv.batch + 64) * 4);
+    kv.rows_dev.ensure((size_t)(4 * kMaxRows + 2 * kv.batch + 64 + kMaxFlashUnits * kUnitWords) * 4);
     if (Mc > 1 && m.wt != DT_F32) kv.gemm_ws.ensure((size_t)256 << 20);  // split-K partials
     if (Mc > 1 && m.wt == DT_F32) {
         // the f32 GEMM's partials: splits keep at least 256 keys
@@ -1573,7 +1594,8 @@ static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, con
     const int lastoff = 3 * kMaxRows;
     const int erroff = lastoff + kv.batch + 8;  // pinned word: the router status read back
     const int grpoff = lastoff + kv.batch + 32;  // row groups of the row attention
-    ensure_pinned(kv, (size_t)(4 * kMaxRows + kv.batch + 64) * 4);
+    const int unitoff = (grpoff + kMaxRows + 7) / 8 * 8;  // flash units of several prompt blocks
+    ensure_pinned(kv, (size_t)(4 * kMaxRows + kv.batch + 64 + kMaxFlashUnits * kUnitWords) * 4);
     // rows of one sequence that the matrix-core row attention serves per wave
     const int G = m.nq / m.nkv, grp_rows = G >= 1 && G <= 16 ? 16 / G : 1;
     if (kv.moe_err.p) launch_fill_const(kv.moe_err.as<float>(), 1, 0.f, s);
@@ -1592,6 +1614,7 @@ static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, con
         // cut into row groups of up to grp_rows rows
         std::vector<Seg> segs;
         int ngrp = 0;
+        FlashUnits units;
         if (n_seqs > 1) {
             for (int r = 0; r < Mc; ++r) {
                 const long long g = c0 + r;
@@ -1603,8 +1626,12 @@ static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, con
             for (const Seg &sg : segs)
                 for (int r = 0; r < sg.len; r += grp_rows)
                     pin[grpoff + ngrp++] = (sg.row0 + r) | (std::min(grp_rows, sg.len - r) << 16);
+            units.n = flash_units(segs, (FlashUnit *)(pin + unitoff));
+            units.dev = (const FlashUnit *)(dev + unitoff);
         }
-        ESP_HIP(hipMemcpyAsync(dev, pin, (size_t)(ngrp ? grpoff + ngrp : lastoff + n_seqs) * 4,
+        ESP_HIP(hipMemcpyAsync(dev, pin,
+                               (size_t)(units.n ? unitoff + units.n * kUnitWords
+                                                : ngrp ? grpoff + ngrp : lastoff + n_seqs) * 4,
                                hipMemcpyHostToDevice, s));
         Rows rows{dev, dev + kMaxRows, dev + 2 * kMaxRows, Mc, n_seqs == 1 ? (int)seqs[0] : -1};
         if (ngrp) {
@@ -1613,8 +1640,8 @@ static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, con
             rows.grp_rows = grp_rows;
         }
         const bool normed = embed_rows(m, kv, rows.ids, Mc);
-        if (n_seqs == 1) run_layers(m, kv, rows, Mc, max_t, (int)seqs[0], rpos[c0], nullptr, normed);
-        else run_layers(m, kv, rows, Mc, max_t, -1, 0, &segs, normed);
+        if (n_seqs == 1) run_layers(m, kv, rows, Mc, max_t, (int)seqs[0], rpos[c0], {}, normed);
+        else run_layers(m, kv, rows, Mc, max_t, -1, 0, units, normed);
         if (one_chunk) break;
         // keep the hidden state of every sequence's last row in this chunk
         for (int i = 0; i < n_seqs; ++i)

@@ -53,3 +53,25 @@ def test_packed_rows(bits, hidden, ffn, rows):
     shapes = {n: a.shape for n, (a, _) in tensors.items()}
     ref = oracle.OracleModel(cfg, quant.dequantized_model(art, shapes, bits))
     _rows_match(DecoderModel.from_bytes(cfg, st.dump(art), f"q{bits}-block32"), ref, 131, rows, 1e-4)
+
+
+@pytest.mark.parametrize("kv", ["f32", "f16"])
+@pytest.mark.parametrize("lens", [(16, 128, 129), (257, 16, 31, 400), (1100, 20), (2050, 2049, 40)])
+def test_prompt_blocks_in_one_launch(kv, lens):
+    """Several sequences' prompt blocks of 16 rows or more attend in one launch
+    (edges of 128-row query blocks and their pairs; the last case crosses a
+    4096-row chunk): each sequence's logits are those of its prompt alone,
+    whose projections split K elsewhere, within the bf16 path's rounding."""
+    print(f"prompt blocks {lens} {kv}", flush=True)
+    cfg = synth.llama_config(2, 256, 4, 2, 512, 300, head_dim=64, max_pos=4096)
+    model = DecoderModel.synthetic(cfg, seed=3, std=0.05, fmt="bf16")
+    blocks = [synth.uniform_ids(11 + i, n, 300) for i, n in enumerate(lens)]
+    cache = model.new_cache(len(lens), max(lens) + 1, kv)
+    got = model.forward_batch(cache, list(range(len(lens))), blocks)
+    one = model.new_cache(1, max(lens) + 1, kv)
+    tol = 1e-4 if kv == "f32" else 2e-3  # a half-precision cache rounds other last bits
+    for r, b in enumerate(blocks):
+        one.reset(0)
+        want = model.try_forward_cached_last(b, one)
+        err = float(np.abs(got[r] - want).max())
+        assert err <= tol * float(np.abs(want).max()), f"sequence {r} of {lens}: {err}"
