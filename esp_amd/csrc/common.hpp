@@ -119,6 +119,9 @@ struct GemmArgs {
     const int32_t *grp_offs;
     int grp_n;
     long long grp_w_stride;
+    // Nullable (device): row m of the product is row a_rows[m] of A, which then
+    // need not be gathered first. Only where gemm_takes_rows says so.
+    const int32_t *a_rows;
     // Nullable host word. When set, a launch that splits K leaves the
     // partial sums in ws ([splits][M][N] f32) and stores the split count
     // here instead of running the reduction and epilogue (the consumer sums
@@ -134,6 +137,8 @@ struct GemmArgs {
     int band;
 };
 void launch_gemm(Dt wt, GemmEpi epi, const GemmArgs &a, hipStream_t s);
+// Whether launch_gemm takes a_rows for these operands.
+bool gemm_takes_rows(Dt wt, const GemmArgs &a);
 
 // QKV post-processing: LoRA B-adds, optional QK RMSNorm, RoPE at each row's
 // position, K/V append into the cache, q written as f32 [M, nq, hd].

@@ -128,18 +128,18 @@ __device__ void route_row_wave(const RouteArgs &a, int t, float *pr, int *ssel =
     }
 }
 
-// Decode-sized routing (up to 16 rows, 64 selections and 64 experts): one
-// wave takes the rows in turn and then groups the selections from its LDS
-// copy with ballots (counts per expert, ranks from the lanes below), the
-// same offsets, grouped rows and tokens as route_group.
-__global__ void __launch_bounds__(64) route_small_k(RouteArgs a) {
-    __shared__ float pr[64];
+// Decode-sized routing (up to 16 rows, 64 selections and 64 experts): a wave
+// per row (one wave taking six rows in turn: 23 us), then the first wave
+// groups the selections from the LDS copy with ballots (counts per expert,
+// ranks from the lanes below), the same offsets, grouped rows and tokens as
+// route_group.
+__global__ void __launch_bounds__(1024) route_small_k(RouteArgs a) {
+    __shared__ float pr[16][64];
     __shared__ int ssel[64];
-    const int lane = threadIdx.x, E = a.E, k = a.k, R = a.M * k;
-    for (int t = 0; t < a.M; ++t) route_row_wave(a, t, pr, ssel);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, E = a.E, k = a.k, R = a.M * k;
+    route_row_wave(a, wave, pr[wave], ssel);
+    __syncthreads();
+    if (wave) return;
     const int sv = lane < R ? ssel[lane] : E;  // E: no selection
     int status = max(0, -sv);
     for (int o = 32; o >= 1; o >>= 1) status = max(status, __shfl_xor(status, o, 64));
@@ -367,7 +367,7 @@ __global__ void __launch_bounds__(256) route_k(RouteArgs a) {
 void launch_route(const RouteArgs &a, hipStream_t s) {
     if (a.E > 256 || a.k > 8) fail(ESP_UNSUPPORTED, "config.experts: more than 256 experts or top-k above 8");
     if (a.M <= 16 && a.M * a.k <= 64 && a.E <= 64) {
-        route_small_k<<<1, 64, 0, s>>>(a);
+        route_small_k<<<1, 64 * a.M, 0, s>>>(a);
         return;
     }
     if (a.M <= 256) {
@@ -378,18 +378,31 @@ void launch_route(const RouteArgs &a, hipStream_t s) {
     route_group_k<<<1, 256, 0, s>>>(a);
 }
 
+// `planes` matrices of src_plane elements each (hi and lo), 16 bytes a thread
+// where the rows allow it
 template <typename T>
-__global__ void __launch_bounds__(256) gather_k(const T *src, const int32_t *perm, int H, T *dst) {
-    int r = blockIdx.x;
-    const T *s = src + (size_t)perm[r] * H;
-    for (int j = threadIdx.x; j < H; j += blockDim.x) dst[(size_t)r * H + j] = s[j];
+__global__ void __launch_bounds__(256) gather_k(const T *src, size_t src_plane, const int32_t *perm, int H,
+                                                T *dst) {
+    const int r = blockIdx.x;
+    const T *s = src + blockIdx.y * src_plane + (size_t)perm[r] * H;
+    T *d = dst + ((size_t)blockIdx.y * gridDim.x + r) * H;
+    for (int j = threadIdx.x; j < H; j += blockDim.x) d[j] = s[j];
 }
 
-void launch_gather_rows(Dt dt, const void *src, const int32_t *perm, int rows, int H, void *dst,
+void launch_gather_rows(Dt dt, int src_rows, const void *src, const int32_t *perm, int rows, int H, void *dst,
                         hipStream_t s) {
     if (!rows) return;
-    if (dt == DT_BF16) gather_k<uint16_t><<<rows, 256, 0, s>>>((const uint16_t *)src, perm, H, (uint16_t *)dst);
-    else gather_k<float><<<rows, 256, 0, s>>>((const float *)src, perm, H, (float *)dst);
+    const int planes = dt == DT_SPLIT ? 2 : 1;
+    const size_t bytes = (size_t)H * (dt == DT_F32 ? 4 : 2);
+    if (bytes % 16 == 0 && (uintptr_t)src % 16 == 0 && (uintptr_t)dst % 16 == 0) {
+        const int h = (int)(bytes / 16);
+        gather_k<uint4><<<dim3(rows, planes), std::min(256, (h + 63) / 64 * 64), 0, s>>>(
+            (const uint4 *)src, (size_t)src_rows * h, perm, h, (uint4 *)dst);
+    } else if (dt == DT_SPLIT) {
+        gather_k<uint16_t><<<dim3(rows, 2), 256, 0, s>>>((const uint16_t *)src, (size_t)src_rows * H, perm, H, (uint16_t *)dst);
+    } else {
+        gather_k<float><<<rows, 256, 0, s>>>((const float *)src, 0, perm, H, (float *)dst);
+    }
 }
 
 // One thread per (token, hidden element): every load of a thread is

@@ -35,7 +35,9 @@ struct RouteArgs {
     const int32_t *step;
 };
 void launch_route(const RouteArgs &a, hipStream_t s);
-void launch_gather_rows(Dt dt, const void *src, const int32_t *perm, int rows, int H, void *dst,
+// dst[r] = src[perm[r]]: f32 rows, or both planes of a DT_SPLIT matrix of
+// src_rows rows (dst: planes of `rows` rows).
+void launch_gather_rows(Dt dt, int src_rows, const void *src, const int32_t *perm, int rows, int H, void *dst,
                         hipStream_t s);
 struct CombineArgs {
     const float *y;      // [M * k, H] grouped expert outputs
@@ -48,7 +50,7 @@ struct CombineArgs {
 };
 void launch_combine(const CombineArgs &a, hipStream_t s);
 
-void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l);
+void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_splits = 0);
 // one decode row through the routed experts without host round trips
 bool moe_decode_ok(const Model &m);
 void moe_decode(Model &m, Kv &kv, LayerW &w, hipStream_t s);

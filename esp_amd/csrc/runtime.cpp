@@ -1308,13 +1308,13 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
             g.N = H;
             g.K = m.qw;
             g.ldc = H;
-            if (!w.moe && resid_norm_ok(H)) g.defer_splits = &o_splits;
+            if (resid_norm_ok(H)) g.defer_splits = &o_splits;
             Prof p("gemm_o", s);
             launch_gemm(m.wt, GEMM_RESIDUAL, g, s);
         }
         // ---- MLP block (layer.rs:147-151)
         if (w.moe) {
-            moe_block(m, kv, w, Mc, s, l);
+            moe_block(m, kv, w, Mc, s, l, o_splits);
         } else if (single) {
             GemvArgs g{};
             g.w = w.gate;
@@ -1892,11 +1892,16 @@ void moe_decode(Model &m, Kv &kv, LayerW &w, hipStream_t s) {
 // round trip: the expert GEMMs are one grouped launch each over all experts,
 // their row ranges read from the router's offsets on the device, so the
 // block can be captured. A router failure is reported at the forward's end.
-void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l) {
+// o_splits: the o_proj partial sums of that many k splits still to be added.
+void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_splits) {
     const Dt act = m.wt == DT_BF16 ? DT_SPLIT : DT_F32;
     const bool split = act == DT_SPLIT;
     const int H = m.H, E = m.E, k = m.topk, R = Mc * k;
-    {
+    if (o_splits > 1) {
+        Prof p("resid_norm", s);
+        launch_resid_norm(kv.gemm_ws.as<float>(), o_splits, Mc, H, w.o_bias, kv.h.as<float>(), w.post_norm,
+                          m.cfg.rms_norm_eps, act, kv.xn.p, s);
+    } else {
         Prof p("rmsnorm", s);
         launch_rmsnorm(kv.h.as<float>(), w.post_norm, m.cfg.rms_norm_eps, Mc, H, act, kv.xn.p,
                        nullptr, s);
@@ -1933,15 +1938,6 @@ void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l) {
     {
         Prof p("moe", s);
         launch_route(ra, s);
-        if (split) {
-            const uint16_t *xs = kv.xn.as<uint16_t>();
-            uint16_t *xd = kv.moe_x.as<uint16_t>();
-            launch_gather_rows(DT_BF16, xs, kv.moe_perm.as<int32_t>(), R, H, xd, s);
-            launch_gather_rows(DT_BF16, xs + (size_t)Mc * H, kv.moe_perm.as<int32_t>(), R, H,
-                               xd + (size_t)R * H, s);
-        } else {
-            launch_gather_rows(DT_F32, kv.xn.p, kv.moe_perm.as<int32_t>(), R, H, kv.moe_x.p, s);
-        }
     }
     const size_t es = split ? 2 : 4;  // bytes per element of one plane
     char *xh = (char *)kv.moe_x.p, *ah = (char *)kv.moe_act.p;
@@ -1975,6 +1971,15 @@ void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l) {
     d.grp_offs = g.grp_offs;
     d.grp_n = E;
     d.grp_w_stride = (long long)H * m.Fe;
+    // the few-row form reads the tokens' rows through the grouping itself
+    if (w.ex_gate && gemm_takes_rows(m.wt, g)) {
+        g.a = kv.xn.p;
+        g.a_lo = lo_plane(act, kv.xn, Mc, H);
+        g.a_rows = kv.moe_perm.as<int32_t>();
+    } else {
+        Prof p("moe", s);
+        launch_gather_rows(act, Mc, kv.xn.p, kv.moe_perm.as<int32_t>(), R, H, kv.moe_x.p, s);
+    }
     if (w.ex_gate) {
         Prof p("gemm", s);
         launch_gemm(m.wt, GEMM_SWIGLU, g, s);

@@ -7,7 +7,7 @@ sequence attends to itself only, so the oracle evaluates each id once.
 import numpy as np
 import pytest
 
-from esp_amd import DecoderModel
+from esp_amd import DecoderConfig, DecoderModel
 from oracle import oracle, quant, st
 from tests import synth
 
@@ -75,3 +75,31 @@ def test_prompt_blocks_in_one_launch(kv, lens):
         want = model.try_forward_cached_last(b, one)
         err = float(np.abs(got[r] - want).max())
         assert err <= tol * float(np.abs(want).max()), f"sequence {r} of {lens}: {err}"
+
+
+# K 128 (one group), 256, 640 (a ragged chunk of 512) and, with k splits, 1152
+@pytest.mark.parametrize("hidden,ffn", [(128, 256), (256, 640), (512, 1152)])
+@pytest.mark.parametrize("rows", [2, 4, 5, 8, 9, 15, 16])
+def test_bf16_few_rows(hidden, ffn, rows):
+    """bf16 weights over few rows, on both sides of the few-row form's end
+    (15): 1e-4 of the row's magnitude (activations as two bf16 halves)."""
+    print(f"bf16 rows {rows} hidden {hidden} ffn {ffn}", flush=True)
+    cfg = synth.llama_config(2, hidden, 4, 2, ffn, 131, head_dim=32 if hidden < 512 else 64)
+    tensors = synth.make_tensors(cfg, 9, "bf16", std=0.05)
+    ref = oracle.OracleModel(cfg, tensors)
+    _rows_match(DecoderModel.from_bytes(cfg, st.dump(tensors), "bf16"), ref, 131, rows, 1e-4)
+
+
+# rows per expert on average: 1, 3, 8, 20, 48 and past each
+@pytest.mark.parametrize("rows", [2, 6, 7, 16, 17, 40, 42, 96, 100])
+def test_bf16_moe_rows(rows):
+    """Routed experts over few rows: grouped few-row products whose tiles end
+    inside and between the experts' rows, read through the router's grouping."""
+    print(f"moe rows {rows}", flush=True)
+    cfg = DecoderConfig.mixtral_style(vocab_size=131, hidden_size=256, intermediate_size=384,
+                                      num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2,
+                                      max_position_embeddings=64, num_experts=4, num_experts_per_tok=2,
+                                      moe_intermediate_size=384)
+    tensors = synth.make_tensors(cfg, 9, "bf16", std=0.05)
+    ref = oracle.OracleModel(cfg, tensors)
+    _rows_match(DecoderModel.from_bytes(cfg, st.dump(tensors), "bf16"), ref, 131, rows, 1e-4)
