@@ -1481,7 +1481,9 @@ static void run_head(Model &m, Kv &kv, int n_seqs, const float *h_src, const int
         g.y = kv.logits.as<float>();
         g.N = m.V;
         g.K = m.H;
-        g.ticket = t + kHeadTicket;
+        // the fused argmax only where the device loop takes it: its merge over
+        // the head's blocks costs ~8 us (pick reads the logits)
+        g.ticket = gen ? t + kHeadTicket : nullptr;
         g.part_v = (float *)(t + kHeadTicket + 8);
         g.part_i = t + kHeadTicket + 8 + DG_MAX_PART;
         g.picked = (uint32_t *)(t + kHeadTicket + 8 + 2 * DG_MAX_PART);
