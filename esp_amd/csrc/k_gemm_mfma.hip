@@ -1079,6 +1079,13 @@ template <int EPI> static void mfma_launch(const GemmArgs &a, float *ws, size_t 
     // long row counts (prefill of >= 1024 tokens) take the LDS-streamed form:
     // 256-row blocks for one weight matrix, 128-row blocks for gate/up pairs
     if (a.K % LS_BK == 0 && a.M >= 1024) {
+        // Routed groups fill 256-row tiles badly and leave most CUs without
+        // one: the down projection takes 128-row tiles like gate/up (eight
+        // experts of 2048 x 7168: 1554 rows 202 -> 175 us, 4096 rows 375 -> 333)
+        if (NB == 1 && a.grp_offs) {
+            lds_launch<EPI, NB, 2>(a, ws, ws_bytes, s, 2 * g_cus);
+            return;
+        }
         if (NB == 1) lds_launch<EPI, NB, 4>(a, ws, ws_bytes, s, g_cus);
         else lds_launch<EPI, NB, 2>(a, ws, ws_bytes, s, 2 * g_cus);
         return;
