@@ -279,12 +279,6 @@ esp_status esp_kv_logits(esp_kv *kv, float **rows_dev, uint32_t *n_rows) {
 }
 
 // the forward may still be in flight on the handle's (non-blocking) stream
-static void copy_logits(Kv &kv, int rows, float *out) {
-    if (!out) return;
-    ESP_HIP(hipMemcpyAsync(out, kv.logits.p, (size_t)rows * kv.model->V * 4, hipMemcpyDeviceToHost, kv.stream));
-    ESP_HIP(hipStreamSynchronize(kv.stream));
-}
-
 esp_status esp_forward_last(esp_model *model, esp_kv *kv, uint32_t seq, const int32_t *ids,
                             uint32_t n, float *logits_out) {
     return guard([&] {
@@ -293,8 +287,7 @@ esp_status esp_forward_last(esp_model *model, esp_kv *kv, uint32_t seq, const in
         if (!n || !ids) fail(ESP_INVALID_REQUEST, "cached input is empty or exceeds the context window");
         Kv &k = *(Kv *)kv;
         if (k.model != (Model *)model) fail(ESP_INVALID_REQUEST, "kv handle belongs to another model");
-        forward(*(Model *)model, k, 1, &seq, &n, ids);
-        copy_logits(k, 1, logits_out);
+        forward(*(Model *)model, k, 1, &seq, &n, ids, logits_out);
     });
 }
 
@@ -307,8 +300,7 @@ esp_status esp_forward_batch(esp_model *model, esp_kv *kv, uint32_t n_seqs, cons
             fail(ESP_INVALID_REQUEST, "cached input is empty or exceeds the context window");
         Kv &k = *(Kv *)kv;
         if (k.model != (Model *)model) fail(ESP_INVALID_REQUEST, "kv handle belongs to another model");
-        forward(*(Model *)model, k, (int)n_seqs, seqs, seq_lens, ids);
-        copy_logits(k, (int)n_seqs, logits_out);
+        forward(*(Model *)model, k, (int)n_seqs, seqs, seq_lens, ids, logits_out);
     });
 }
 

@@ -32,6 +32,7 @@ struct Rows;
 Kv::~Kv() {
     if (gen_exec) (void)hipGraphExecDestroy(gen_exec);
     if (pinned) (void)hipHostFree(pinned);
+    if (logits_pin) (void)hipHostFree(logits_pin);
     if (pick_pinned) (void)hipHostFree(pick_pinned);
     if (pick_up) (void)hipEventDestroy(pick_up);
     if (pick_stream) (void)hipStreamDestroy(pick_stream);
@@ -764,14 +765,18 @@ static void *kv_layer(Kv &kv, int l) {
 
 static constexpr int kMaxRows = 4096;  // token rows per pass through the layers
 
-static void ensure_pinned(Kv &kv, size_t bytes) {
-    if (kv.pinned_bytes >= bytes) return;
-    if (kv.pinned) ESP_HIP(hipHostFree(kv.pinned));
-    kv.pinned = nullptr;
-    kv.pinned_bytes = 0;
-    ESP_HIP(hipHostMalloc(&kv.pinned, bytes, hipHostMallocDefault));
-    kv.pinned_bytes = bytes;
+// A grow-only pinned host buffer; nothing in flight may use it.
+static void ensure_host(void *&p, size_t &have, size_t bytes) {
+    if (have >= bytes) return;
+    if (p) ESP_HIP(hipHostFree(p));
+    p = nullptr;
+    have = 0;
+    ESP_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+    have = bytes;
 }
+static void ensure_pinned(Kv &kv, size_t bytes) { ensure_host(kv.pinned, kv.pinned_bytes, bytes); }
+
+static constexpr size_t kLogitsPin = (size_t)1 << 20;  // most logits bytes returned through pinned memory
 
 struct Plan {
     int n_split, split_len;
@@ -1075,6 +1080,11 @@ constexpr int kMinFlashSeg = 16;
 // a segment of len >= 16 rows has at most 1 + len / 256 pairs
 constexpr int kMaxFlashUnits = kMaxRows / kMinFlashSeg + kMaxRows / 256;
 constexpr int kUnitWords = sizeof(FlashUnit) / 4;
+
+// 32-bit words of a chunk's row descriptors (forward_pass) at their largest
+static int rows_words(const Kv &kv) {
+    return 4 * kMaxRows + kv.batch + kMaxFlashUnits * kUnitWords + 4 * 64;
+}
 
 // Writes the units of `segs` (longest key range first, so that the last ones
 // to start are short) to `out`; 0 if a segment is shorter than 16 rows.
@@ -1410,7 +1420,7 @@ static void ensure_scratch(Model &m, Kv &kv, int Mc, int n_seqs) {
     kv.act.ensure((size_t)Mc * fmax * 4);
     kv.last_h.ensure((size_t)n_seqs * H * 4);
     kv.logits.ensure((size_t)std::max(n_seqs, kv.batch) * m.V * 4);
-    kv.rows_dev.ensure((size_t)(4 * kMaxRows + 2 * kv.batch + 64 + kMaxFlashUnits * kUnitWords) * 4);
+    kv.rows_dev.ensure((size_t)rows_words(kv) * 4);
     if (Mc > 1 && m.wt != DT_F32) kv.gemm_ws.ensure((size_t)256 << 20);  // split-K partials
     if (Mc > 1 && m.wt == DT_F32) {
         // the f32 GEMM's partials: splits keep at least 256 keys
@@ -1541,24 +1551,24 @@ bool xcd_merge_failed(Kv &kv) {
 }
 
 static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, const uint32_t *lens,
-                         const int32_t *ids);
+                         const int32_t *ids, float *logits_out);
 
 // One forward; computed again with the agent-scope attention merge when the
 // XCD-local merge's placement check failed (positions only move after a
 // pass that succeeded).
 void forward(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, const uint32_t *lens,
-             const int32_t *ids) {
+             const int32_t *ids, float *logits_out) {
     std::unique_lock<std::recursive_mutex> streaming;
     if (m.st) streaming = std::unique_lock<std::recursive_mutex>(m.st->mu);
     const StreamMark mark = stream_mark(m);
-    if (!forward_pass(m, kv, n_seqs, seqs, lens, ids)) return;
+    if (!forward_pass(m, kv, n_seqs, seqs, lens, ids, logits_out)) return;
     stream_rewind(m, mark);
-    if (forward_pass(m, kv, n_seqs, seqs, lens, ids))
+    if (forward_pass(m, kv, n_seqs, seqs, lens, ids, logits_out))
         fail(ESP_BACKEND, "decode attention: split placement check failed with the agent-scope merge");
 }
 
 static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, const uint32_t *lens,
-                         const int32_t *ids) {
+                         const int32_t *ids, float *logits_out) {
     if (n_seqs <= 0) fail(ESP_INVALID_REQUEST, "cached input is empty or exceeds the context window");
     std::unique_lock<std::recursive_mutex> streaming;
     if (m.st) streaming = std::unique_lock<std::recursive_mutex>(m.st->mu);
@@ -1593,11 +1603,14 @@ static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, con
         }
     }
     hipStream_t s = kv.stream;
-    const int lastoff = 3 * kMaxRows;
-    const int erroff = lastoff + kv.batch + 8;  // pinned word: the router status read back
-    const int grpoff = lastoff + kv.batch + 32;  // row groups of the row attention
-    const int unitoff = (grpoff + kMaxRows + 7) / 8 * 8;  // flash units of several prompt blocks
-    ensure_pinned(kv, (size_t)(4 * kMaxRows + kv.batch + 64 + kMaxFlashUnits * kUnitWords) * 4);
+    // row descriptors of a chunk, packed so that few rows upload few bytes:
+    // ids | sequence | position | last rows | row groups of the row attention
+    // | flash units of several prompt blocks; the last words of the pinned
+    // buffer receive the status words read back
+    auto pad = [](int n) { return (n + 63) / 64 * 64; };
+    const int words = rows_words(kv), erroff = words - 8;
+    ensure_pinned(kv, (size_t)words * 4);
+    int lastoff = 0;
     // rows of one sequence that the matrix-core row attention serves per wave
     const int G = m.nq / m.nkv, grp_rows = G >= 1 && G <= 16 ? 16 / G : 1;
     if (kv.moe_err.p) launch_fill_const(kv.moe_err.as<float>(), 1, 0.f, s);
@@ -1608,14 +1621,16 @@ static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, con
     for (long long c0 = 0; c0 < M; c0 += kMaxRows) {
         int Mc = (int)std::min<long long>(kMaxRows, M - c0);
         ESP_HIP(hipStreamSynchronize(s));  // pinned staging buffer reuse
+        const int mr = pad(Mc), grpoff = 3 * mr + pad(n_seqs);
+        lastoff = 3 * mr;
         memcpy(pin, ids + c0, Mc * 4);
-        memcpy(pin + kMaxRows, rseq.data() + c0, Mc * 4);
-        memcpy(pin + 2 * kMaxRows, rpos.data() + c0, Mc * 4);
+        memcpy(pin + mr, rseq.data() + c0, Mc * 4);
+        memcpy(pin + 2 * mr, rpos.data() + c0, Mc * 4);
         memcpy(pin + lastoff, last.data(), n_seqs * 4);
         // segments: runs of consecutive positions of one sequence; each is
         // cut into row groups of up to grp_rows rows
         std::vector<Seg> segs;
-        int ngrp = 0;
+        int ngrp = 0, used = lastoff + n_seqs;
         FlashUnits units;
         if (n_seqs > 1) {
             for (int r = 0; r < Mc; ++r) {
@@ -1628,14 +1643,13 @@ static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, con
             for (const Seg &sg : segs)
                 for (int r = 0; r < sg.len; r += grp_rows)
                     pin[grpoff + ngrp++] = (sg.row0 + r) | (std::min(grp_rows, sg.len - r) << 16);
+            const int unitoff = grpoff + pad(ngrp);
             units.n = flash_units(segs, (FlashUnit *)(pin + unitoff));
             units.dev = (const FlashUnit *)(dev + unitoff);
+            used = units.n ? unitoff + units.n * kUnitWords : grpoff + ngrp;
         }
-        ESP_HIP(hipMemcpyAsync(dev, pin,
-                               (size_t)(units.n ? unitoff + units.n * kUnitWords
-                                                : ngrp ? grpoff + ngrp : lastoff + n_seqs) * 4,
-                               hipMemcpyHostToDevice, s));
-        Rows rows{dev, dev + kMaxRows, dev + 2 * kMaxRows, Mc, n_seqs == 1 ? (int)seqs[0] : -1};
+        ESP_HIP(hipMemcpyAsync(dev, pin, (size_t)used * 4, hipMemcpyHostToDevice, s));
+        Rows rows{dev, dev + mr, dev + 2 * mr, Mc, n_seqs == 1 ? (int)seqs[0] : -1};
         if (ngrp) {
             rows.grp = dev + grpoff;
             rows.ngrp = ngrp;
@@ -1659,19 +1673,37 @@ static bool forward_pass(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, con
     }
     // The pass is left in flight (later calls on this stream, and reads of
     // the logits, are ordered after it) unless something must be read back:
-    // the router status of MoE layers, a streamed layer's device checks, or
-    // the placement word of a split-merging attention.
-    if (kv.moe_err.p || m.st || kv.att_merged) {
+    // the router status of MoE layers, a streamed layer's device checks, the
+    // placement word of a split-merging attention, or the logits. Up to 1 MB
+    // of logits come back through pinned memory with the same wait as the
+    // status words (a copy to the caller's pageable memory after that wait was
+    // a second one).
+    const size_t lbytes = (size_t)n_seqs * m.V * 4;
+    const bool pin_logits = logits_out && lbytes <= kLogitsPin;
+    const bool status = kv.moe_err.p || m.st || kv.att_merged;
+    if (pin_logits) {
+        ensure_host(kv.logits_pin, kv.logits_pin_bytes, lbytes);
+        ESP_HIP(hipMemcpyAsync(kv.logits_pin, kv.logits.p, lbytes, hipMemcpyDeviceToHost, s));
+    }
+    if (status) {
         if (kv.moe_err.p)
             ESP_HIP(hipMemcpyAsync(pin + erroff, kv.moe_err.p, 4, hipMemcpyDeviceToHost, s));
         ESP_HIP(hipMemcpyAsync(pin + erroff + 1, xcd_err_word(kv), 4, hipMemcpyDeviceToHost, s));
-        ESP_HIP(hipStreamSynchronize(s));
+    }
+    if (status || pin_logits) ESP_HIP(hipStreamSynchronize(s));
+    if (status) {
         if (m.st) stream_check(m);  // a streamed layer that failed its device checks
         if (kv.moe_err.p) moe_fail(pin[erroff]);
         if (pin[erroff + 1] && xcd_merge_failed(kv)) return true;
     }
     for (int i = 0; i < n_seqs; ++i) kv.pos[seqs[i]] += (int)lens[i];
     kv.logits_rows = n_seqs;
+    if (pin_logits) {
+        memcpy(logits_out, kv.logits_pin, lbytes);
+    } else if (logits_out) {
+        ESP_HIP(hipMemcpyAsync(logits_out, kv.logits.p, lbytes, hipMemcpyDeviceToHost, s));
+        ESP_HIP(hipStreamSynchronize(s));
+    }
     return false;
 }
 

@@ -122,6 +122,9 @@ struct Kv {
     bool att_merged = false;
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
+    // logits on their way to the caller; empty again when a call returns
+    void *logits_pin = nullptr;
+    size_t logits_pin_bytes = 0;
     // esp_pick's host staging (masks and samplers in, ids / states / flags
     // out): one DMA each way instead of copies from pageable memory
     void *pick_pinned = nullptr;
@@ -138,9 +141,10 @@ struct Kv {
     ~Kv();
 };
 
-// The forward over prepared rows; defined in runtime.cpp.
+// The forward over prepared rows, its last-position logits copied to
+// logits_out (host, nullable); defined in runtime.cpp.
 void forward(Model &m, Kv &kv, int n_seqs, const uint32_t *seqs, const uint32_t *lens,
-             const int32_t *ids);
+             const int32_t *ids, float *logits_out = nullptr);
 
 // Checkpoint admission rules shared by the resident loader and the layer
 // streamer (runtime.cpp).
