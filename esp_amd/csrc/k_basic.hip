@@ -3,6 +3,7 @@
 // attention over the per-sequence cache.
 #include "common.hpp"
 #include "dev.hpp"
+#include "kernels_extra.hpp"
 
 namespace esp {
 
@@ -82,11 +83,14 @@ __global__ void __launch_bounds__(256) rmsnorm_k(const float *x, const float *ga
 //             from 0 in split order, eight loads in flight, as the GEMM
 //             reduction does
 //   NB_EMBED  x[m] = embedding row ids[m], the first layer's input
+//   NB_COMBINE x[m] += the routed experts' outputs (CombineArgs), before the
+//             next layer's input norm
 // Measured at H 4096, four rows: plain 12.8 -> 4.7 us (was one wave per row),
 // resid 9.2 -> 5.6 us (was 256 threads, a trip per quarter row), embedding and
 // norm 23.4 -> 6.3 us; 2048 rows: resid 32.6 -> 31.7, embedding and norm 43.5
-// -> 26.9 us.
-enum { NB_PLAIN = 0, NB_RESID = 1, NB_EMBED = 2 };
+// -> 26.9 us. H 2048, six rows of two experts: split sums' reduction, combine
+// and norm 3.7 + 6.3 + 4.6 -> 5.3 us.
+enum { NB_PLAIN = 0, NB_RESID = 1, NB_EMBED = 2, NB_COMBINE = 3 };
 struct NormArgs {
     float *x;                  // [M, H] residual stream
     const float *gamma;
@@ -98,7 +102,48 @@ struct NormArgs {
     int splits;
     const void *embed;         // EMBED: [V, H]
     const int32_t *ids;
+    CombineArgs c;             // COMBINE
 };
+
+// Four elements (from j) of row m's combine, in combine_k's order; two
+// experts' rows and four of their split sums in flight.
+__device__ __forceinline__ f32x4 combine4(const CombineArgs &c, int m, int j) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const size_t plane = (size_t)c.M * c.k * c.H;
+    const int ns = max(c.splits, 1);
+    f32x4 out = zero;
+    for (int e0 = 0; e0 < c.k; e0 += 2) {
+        const float *p[2];
+        float wt[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const size_t i = (size_t)m * c.k + min(e0 + q, c.k - 1);
+            p[q] = c.y + (size_t)c.slot[i] * c.H + j;
+            wt[q] = c.w[i];
+        }
+        f32x4 t[2] = {zero, zero};
+        for (int z0 = 0; z0 < ns; z0 += 4) {
+            f32x4 pz[2][4];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int z = 0; z < 4; ++z) pz[q][z] = z0 + z < ns ? *(const f32x4 *)(p[q] + (z0 + z) * plane) : zero;
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int z = 0; z < 4; ++z)
+                    if (z0 + z < ns) t[q] += pz[q][z];
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            if (e0 + q < c.k) out = out + t[q] * wt[q];
+    }
+    if (c.ys) {
+        const float g = 1.0f / (1.0f + expf(-c.sg[m]));
+        out = out + g * *(const f32x4 *)(c.ys + (size_t)m * c.H + j);
+    }
+    return out;
+}
 
 template <bool SPLIT, int NT, int NQ, int MODE, typename ET>
 __global__ void __launch_bounds__(NT) norm_block_k(NormArgs a) {
@@ -136,10 +181,14 @@ __global__ void __launch_bounds__(NT) norm_block_k(NormArgs a) {
             v[i] = v[i] + t;
             *(f32x4 *)(a.x + src + j) = v[i];
         }
+        if (MODE == NB_COMBINE) {
+            v[i] = v[i] + combine4(a.c, m, j);
+            *(f32x4 *)(a.x + src + j) = v[i];
+        }
     }
     // The sum of squares in an order that does not depend on the block's
     // size: every wave adds the quads' sums itself, PLAIN and EMBED as lane l
-    // over quads l + 64 i, RESID as four parts over quads 64 p + l + 256 i.
+    // over quads l + 64 i (COMBINE too), RESID as four parts over quads 64 p + l + 256 i.
 #pragma unroll
     for (int i = 0; i < NQ; ++i)
         sq[tid + NT * i] = v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
@@ -229,6 +278,20 @@ void launch_resid_norm(const float *ws, int splits, int M, int H, const float *b
     a.splits = splits;
     if (out_dt == DT_SPLIT) norm_block<true, NB_RESID, float>(a, s);
     else norm_block<false, NB_RESID, float>(a, s);
+}
+
+void launch_combine_norm(const CombineArgs &c, const float *gamma, float eps, Dt out_dt, void *out, hipStream_t s) {
+    if (!resid_norm_ok(c.H) || (out_dt != DT_SPLIT && out_dt != DT_F32)) fail(ESP_BACKEND, "combine_norm: unsupported shape");
+    NormArgs a{};
+    a.x = c.h;
+    a.gamma = gamma;
+    a.eps = eps;
+    a.M = c.M;
+    a.H = c.H;
+    a.out = out;
+    a.c = c;
+    if (out_dt == DT_SPLIT) norm_block<true, NB_COMBINE, float>(a, s);
+    else norm_block<false, NB_COMBINE, float>(a, s);
 }
 
 bool embed_norm_ok(Dt wt, const void *embed, int H) {

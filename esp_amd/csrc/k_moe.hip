@@ -412,7 +412,9 @@ __global__ void __launch_bounds__(256) combine_k(CombineArgs a) {
     if (d >= a.H) return;
     float out = 0.f;
     for (int j = 0; j < a.k; ++j) {
-        float y = a.y[(size_t)a.slot[(size_t)t * a.k + j] * a.H + d];
+        const float *p = a.y + (size_t)a.slot[(size_t)t * a.k + j] * a.H + d;
+        float y = p[0];
+        for (int z = 1; z < a.splits; ++z) y += p[(size_t)z * a.M * a.k * a.H];
         out = out + y * a.w[(size_t)t * a.k + j];
     }
     if (a.ys) {

@@ -47,10 +47,18 @@ struct CombineArgs {
     const float *sg;     // nullable [M] shared gate logit
     float *h;            // [M, H] residual stream (+=)
     int M, k, H;
+    // y holds that many k-split partial planes still to be summed, in split
+    // order (0 or 1: the outputs themselves)
+    int splits;
 };
 void launch_combine(const CombineArgs &a, hipStream_t s);
+// The combine and out = RMSNorm(h) * gamma (DT_SPLIT planes or f32) in one
+// launch, where resid_norm_ok(H).
+void launch_combine_norm(const CombineArgs &a, const float *gamma, float eps, Dt out_dt, void *out, hipStream_t s);
 
-void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_splits = 0);
+// next_norm (nullable): kv.xn = the following RMSNorm of the block's output too.
+void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_splits = 0,
+               const float *next_norm = nullptr);
 // one decode row through the routed experts without host round trips
 bool moe_decode_ok(const Model &m);
 void moe_decode(Model &m, Kv &kv, LayerW &w, hipStream_t s);

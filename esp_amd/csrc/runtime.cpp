@@ -1324,7 +1324,10 @@ static void run_layers(Model &m, Kv &kv, const Rows &rows, int Mc, int max_t, in
         }
         // ---- MLP block (layer.rs:147-151)
         if (w.moe) {
-            moe_block(m, kv, w, Mc, s, l, o_splits);
+            // the next resident layer's input norm rides the combine
+            const bool next_norm = !single && l + 1 < m.L && !m.st && resid_norm_ok(H);
+            moe_block(m, kv, w, Mc, s, l, o_splits, next_norm ? m.layers[l + 1].in_norm : nullptr);
+            pre_normed = next_norm;
         } else if (single) {
             GemvArgs g{};
             g.w = w.gate;
@@ -1927,7 +1930,7 @@ void moe_decode(Model &m, Kv &kv, LayerW &w, hipStream_t s) {
 // their row ranges read from the router's offsets on the device, so the
 // block can be captured. A router failure is reported at the forward's end.
 // o_splits: the o_proj partial sums of that many k splits still to be added.
-void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_splits) {
+void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_splits, const float *next_norm) {
     const Dt act = m.wt == DT_BF16 ? DT_SPLIT : DT_F32;
     const bool split = act == DT_SPLIT;
     const int H = m.H, E = m.E, k = m.topk, R = Mc * k;
@@ -2014,9 +2017,13 @@ void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_
         Prof p("moe", s);
         launch_gather_rows(act, Mc, kv.xn.p, kv.moe_perm.as<int32_t>(), R, H, kv.moe_x.p, s);
     }
+    int d_splits = 0;
     if (w.ex_gate) {
         Prof p("gemm", s);
         launch_gemm(m.wt, GEMM_SWIGLU, g, s);
+        // the combine takes the down projection's split sums, unless a shared
+        // expert's products use the workspace in between
+        if (!m.Fs) d.defer_splits = &d_splits;
         launch_gemm(m.wt, GEMM_STORE, d, s);
     } else {
         // Streamed experts (moe.rs:183-243): the router's choice comes back
@@ -2056,7 +2063,8 @@ void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_
         }
     }
     CombineArgs c{};
-    c.y = kv.moe_y.as<float>();
+    c.y = d_splits > 1 ? kv.gemm_ws.as<float>() : kv.moe_y.as<float>();
+    c.splits = d_splits;
     c.slot = kv.moe_slot.as<int32_t>();
     c.w = kv.moe_w.as<float>();
     c.h = kv.h.as<float>();
@@ -2109,7 +2117,8 @@ void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_
         c.sg = kv.moe_sg.as<float>();
     }
     Prof p("moe", s);
-    launch_combine(c, s);
+    if (next_norm) launch_combine_norm(c, next_norm, m.cfg.rms_norm_eps, act, kv.xn.p, s);
+    else launch_combine(c, s);
 }
 
 }  // namespace esp

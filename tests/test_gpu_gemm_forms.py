@@ -103,3 +103,18 @@ def test_bf16_moe_rows(rows):
     tensors = synth.make_tensors(cfg, 9, "bf16", std=0.05)
     ref = oracle.OracleModel(cfg, tensors)
     _rows_match(DecoderModel.from_bytes(cfg, st.dump(tensors), "bf16"), ref, 131, rows, 1e-4)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "f32"])
+@pytest.mark.parametrize("rows", [2, 7, 40])
+def test_moe_combine_norm_rows(fmt, rows):
+    """The combine joined with the next layer's norm: an odd number of experts
+    per token, outputs that come as split sums (K 1024 in up to four)."""
+    print(f"moe combine {fmt} rows {rows}", flush=True)
+    cfg = DecoderConfig.mixtral_style(vocab_size=131, hidden_size=256, intermediate_size=1024,
+                                      num_hidden_layers=3, num_attention_heads=4, num_key_value_heads=2,
+                                      max_position_embeddings=64, num_experts=5, num_experts_per_tok=3,
+                                      moe_intermediate_size=1024)
+    tensors = synth.make_tensors(cfg, 11, fmt, std=0.05)
+    ref = oracle.OracleModel(cfg, tensors)
+    _rows_match(DecoderModel.from_bytes(cfg, st.dump(tensors), fmt), ref, 131, rows, 1e-4)
