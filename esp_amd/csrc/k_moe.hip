@@ -69,7 +69,19 @@ __device__ void route_row(const RouteArgs &a, int t) {
 __device__ void route_row_wave(const RouteArgs &a, int t, float *pr, int *ssel = nullptr) {
     const int E = a.E, k = a.k, lane = threadIdx.x & 63;
     const float *l = a.logits + (size_t)t * E;
-    const float x = lane < E ? l[lane] : -INFINITY;
+    float x = lane < E ? l[lane] : -INFINITY;
+    if (a.splits > 1) {  // eight loads in flight
+        x = 0.f;
+        for (int z0 = 0; z0 < a.splits; z0 += 8) {
+            float pz[8];
+#pragma unroll
+            for (int z = 0; z < 8; ++z) pz[z] = lane < E && z0 + z < a.splits ? l[(size_t)(z0 + z) * a.M * E + lane] : 0.f;
+#pragma unroll
+            for (int z = 0; z < 8; ++z)
+                if (z0 + z < a.splits) x += pz[z];
+        }
+        if (lane >= E) x = -INFINITY;
+    }
     float mx = -INFINITY;
     for (int e = 0; e < E; ++e) mx = fmaxf(mx, __shfl(x, e, 64));
     const float ex = lane < E ? expf(x - mx) : 0.f;
@@ -361,10 +373,17 @@ __global__ void __launch_bounds__(256) route_k(RouteArgs a) {
     route_group(a);
 }
 
+// Rows routed by a wave each read every logit once, so the router projection's
+// split sums are added there (a launch less per layer: two routed layers over
+// six rows 475 -> 468 us); the
+// other forms read a logit several times.
+bool route_takes_splits(int M, int E) { return M <= 16 && E <= 64; }
+
 // More rows: the rows' top-k over the grid, one row per thread (one block
 // walking the 2048 rows of a MoE prefill layer took 134 us), then the
 // grouping in one block.
 void launch_route(const RouteArgs &a, hipStream_t s) {
+    if (a.splits > 1 && !route_takes_splits(a.M, a.E)) fail(ESP_BACKEND, "router: split logits outside the wave form");
     if (a.E > 256 || a.k > 8) fail(ESP_UNSUPPORTED, "config.experts: more than 256 experts or top-k above 8");
     if (a.M <= 16 && a.M * a.k <= 64 && a.E <= 64) {
         route_small_k<<<1, 64 * a.M, 0, s>>>(a);

@@ -33,7 +33,12 @@ struct RouteArgs {
     // nullable: the device generation loop's step counter (emitted tokens so
     // far); a failing route then also records min(step << 2 | status) in err[1]
     const int32_t *step;
+    // logits holds that many k-split partial planes still to be summed, in
+    // split order (0 or 1: the logits themselves); more only where
+    // route_takes_splits
+    int splits;
 };
+bool route_takes_splits(int M, int E);
 void launch_route(const RouteArgs &a, hipStream_t s);
 // dst[r] = src[perm[r]]: f32 rows, or both planes of a DT_SPLIT matrix of
 // src_rows rows (dst: planes of `rows` rows).

@@ -1965,13 +1965,15 @@ void moe_block(Model &m, Kv &kv, LayerW &w, int Mc, hipStream_t s, int l, int o_
     // it over the chip (2048 rows: 186 -> 32 us)
     r.ws = kv.gemm_ws.as<float>();
     r.ws_bytes = kv.gemm_ws.bytes;
+    int r_splits = 0;
+    if (route_takes_splits(Mc, E)) r.defer_splits = &r_splits;
     {
         Prof p("gemm", s);
         launch_gemm(m.wt, GEMM_STORE, r, s);
     }
-    RouteArgs ra{kv.moe_logits.as<float>(), Mc, E, k, m.norm_topk ? 1 : 0,
+    RouteArgs ra{r_splits > 1 ? kv.gemm_ws.as<float>() : kv.moe_logits.as<float>(), Mc, E, k, m.norm_topk ? 1 : 0,
                  kv.moe_sel.as<int32_t>(), kv.moe_w.as<float>(), kv.moe_offs.as<int32_t>(),
-                 kv.moe_perm.as<int32_t>(), kv.moe_slot.as<int32_t>(), moe_err_word(kv), kv.gen_step};
+                 kv.moe_perm.as<int32_t>(), kv.moe_slot.as<int32_t>(), moe_err_word(kv), kv.gen_step, r_splits};
     {
         Prof p("moe", s);
         launch_route(ra, s);
