@@ -278,7 +278,6 @@ esp_status esp_kv_logits(esp_kv *kv, float **rows_dev, uint32_t *n_rows) {
     });
 }
 
-// the forward may still be in flight on the handle's (non-blocking) stream
 esp_status esp_forward_last(esp_model *model, esp_kv *kv, uint32_t seq, const int32_t *ids,
                             uint32_t n, float *logits_out) {
     return guard([&] {
