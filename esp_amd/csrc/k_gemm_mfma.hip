@@ -1019,8 +1019,17 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2,
         }
 }
 
-// k split as for the streamed form; each split's range is a multiple of
-// D stages (K % (32 D) == 0 is checked by the caller)
+// k split as for the streamed form
+static int skinny_splits(const GemmArgs &a, int gx, int NB, size_t ws_bytes, int want_blocks, int min_ks) {
+    int splits = 1;
+    while (gx * splits < want_blocks && a.K / (splits * 2) >= min_ks &&
+           (size_t)(splits * 2) * NB * a.M * a.N * 4 <= ws_bytes)
+        splits *= 2;
+    return splits;
+}
+
+// each split's range is a multiple of D stages (K % (32 D) == 0 is checked by
+// the caller)
 template <int EPI, int NB, int RB, int NW, int D>
 static void skinny_launch(const GemmArgs &a, float *ws, size_t ws_bytes, hipStream_t s,
                           int want_blocks, int min_ks) {
@@ -1036,10 +1045,7 @@ static void skinny_launch(const GemmArgs &a, float *ws, size_t ws_bytes, hipStre
     constexpr int BN = 32 * NW, KU = LS_BK * D;
     if (a.K % KU != 0 || a.M > 32 * RB) fail(ESP_BACKEND, "skinny GEMM: shape outside the form");
     const int gx = (a.N + BN - 1) / BN;
-    int splits = 1;
-    while (gx * splits < want_blocks && a.K / (splits * 2) >= min_ks &&
-           (size_t)(splits * 2) * NB * a.M * a.N * 4 <= ws_bytes)
-        splits *= 2;
+    int splits = skinny_splits(a, gx, NB, ws_bytes, want_blocks, min_ks);
     int kps = (a.K + splits - 1) / splits;
     kps = (kps + KU - 1) / KU * KU;
     splits = (a.K + kps - 1) / kps;
@@ -1061,6 +1067,15 @@ static void init_cus() {
     ESP_HIP(hipGetDevice(&dev));
     ESP_HIP(hipDeviceGetAttribute(&g_cus, hipDeviceAttributeMultiprocessorCount, dev));
     if (g_cus <= 0) g_cus = 256;
+}
+
+// The blocks of a skinny streamed launch (128 columns per matrix, k splits)
+// against the CUs: more (1), as many (0) or fewer (-1).
+int gemm_skinny_rounds(const GemmArgs &a) {
+    init_cus();
+    const int gx = (a.N + 127) / 128;
+    const int blocks = gx * skinny_splits(a, gx, a.w2 ? 2 : 1, a.ws ? a.ws_bytes : 0, g_cus, 256);
+    return blocks > g_cus ? 1 : blocks == g_cus ? 0 : -1;
 }
 
 void launch_gemm_reduce(GemmEpi epi, const GemmArgs &a, const float *ws, int splits, hipStream_t s) {

@@ -21,6 +21,8 @@
 
 namespace esp {
 
+int gemm_skinny_rounds(const GemmArgs &a);  // k_gemm_mfma.hip
+
 typedef __bf16 bf16x8r_t __attribute__((ext_vector_type(8)));
 typedef float f32x4r_t __attribute__((ext_vector_type(4)));
 typedef const void __attribute__((address_space(1))) *grptr_t;
@@ -175,13 +177,30 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ROWS <
     }
 }
 
+// Dense launches (2 - 15 rows) that the skinny streamed form, 128 columns and
+// one k range a block, does not do better. Where its blocks fill one round of
+// the CUs or less it keeps up: a block's whole range is then in flight from
+// the start. Past one round the last round is ragged; gate/up below a round
+// gets twice the blocks here; and from 96 MB on the resident activations pay.
+// us per launch (events around it), skinny -> here, at 2 and 14 rows: o of the 1B shape (128
+// blocks) 7.9 -> 7.9, 8.1 -> 8.9, its gate/up (256, 67 MB) 20.2 -> 20.0, 21.4 ->
+// 22.9, down (256, 34 MB) 12.9 -> 13.6, 13.0 -> 15.2; 8B-shape q/k/v (384
+// blocks) 19.0 -> 15.4, 19.4 -> 17.5, gate/up (448) 61.7 -> 53.6, 62.8 -> 58.4,
+// down (256, 117 MB) 32.4 -> 29.7, 34.9 -> 33.0; gate/up of 1024 x 2816 (88)
+// 13.6 -> 11.4, 14.0 -> 12.5; gate/up of 3072 x 8192 (256, 101 MB) 33 -> 28, 33.3
+// -> 31.6.
+static bool dense_rows(const GemmArgs &a) {
+    const int nb = a.w2 ? 2 : 1, rounds = gemm_skinny_rounds(a);
+    return rounds > 0 || (nb == 2 && rounds < 0) || (long long)nb * a.N * a.K * 2 >= 96000000;
+}
+
 // Rows per tile; 0: not this form. Dense launches of at most 15 rows (a
 // decoding batch or forced span of 16 rows and more has a form of its own:
 // gemm_skinny_k, gemm_lds_k); grouped launches of up to 48 rows per group on
 // average, whose groups' weights are read once per tile.
 static int rows_tile(const GemmArgs &a) {
     if (a.K % GR_GK) return 0;
-    if (!a.grp_offs) return a.M <= 4 ? 4 : a.M <= 8 ? 8 : a.M < 16 ? 16 : 0;
+    if (!a.grp_offs) return a.M >= 16 || !dense_rows(a) ? 0 : a.M <= 4 ? 4 : a.M <= 8 ? 8 : 16;
     const int avg = (a.M + a.grp_n - 1) / a.grp_n;
     return a.M <= 4 ? 4 : avg <= 3 ? 8 : avg <= 8 ? 16 : avg <= 20 ? 32 : avg <= 48 ? 64 : 0;
 }
@@ -200,11 +219,14 @@ template <int EPI, int NB, int ROWS> static void rows_launch(const GemmArgs &a, 
     }
     constexpr int BN = 128 / NB;
     const int gx = (a.N + BN - 1) / BN, gy = (a.M + ROWS - 1) / ROWS + (a.grp_offs ? a.grp_n : 0);
-    // K splits until three blocks per CU (the groups' tiles counted as one per
-    // group that can have a row), in ranges of at least 256 keys
+    // K splits of at least 256 keys until two blocks per CU; grouped launches
+    // until three, the groups' tiles counted as one per group that can have a
+    // row. (Three for dense ones cost more in chunk refills and partial sums:
+    // 8B-shape down at 4 rows 33.1 -> 30.1 us, 1B-shape 8-row pass -1.5%.)
+    const int want = (a.grp_offs ? 3 : 2) * cus;
     const long long tiles = (long long)gx * (a.grp_offs ? std::min(a.grp_n, a.M) : 1);
     int splits = 1;
-    while (tiles * splits < 3 * cus && a.K / (splits * 2) >= 256 && a.ws &&
+    while (tiles * splits < want && a.K / (splits * 2) >= 256 && a.ws &&
            (size_t)(splits * 2) * NB * a.M * a.N * 4 <= a.ws_bytes)
         splits *= 2;
     const int kps = ((a.K + splits - 1) / splits + GR_GK - 1) / GR_GK * GR_GK;

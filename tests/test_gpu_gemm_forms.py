@@ -77,15 +77,20 @@ def test_prompt_blocks_in_one_launch(kv, lens):
         assert err <= tol * float(np.abs(want).max()), f"sequence {r} of {lens}: {err}"
 
 
-# K 128 (one group), 256, 640 (a ragged chunk of 512) and, with k splits, 1152
-@pytest.mark.parametrize("hidden,ffn", [(128, 256), (256, 640), (512, 1152)])
+# The narrow shapes take the few-row form for gate/up only (K 128, 256 and 512:
+# its k ranges are a group or two); hidden 4224 takes it everywhere (33, 55 and
+# more column blocks with k splits, more than one round of 256 CUs).
+@pytest.mark.parametrize("hidden,ffn,heads,kv_heads", [(128, 256, 4, 2), (256, 640, 8, 2), (512, 1152, 8, 2),
+                                                       (4224, 2048, 33, 11)])
 @pytest.mark.parametrize("rows", [2, 4, 5, 8, 9, 15, 16])
-def test_bf16_few_rows(hidden, ffn, rows):
-    """bf16 weights over few rows, on both sides of the few-row form's end
-    (15): 1e-4 of the row's magnitude (activations as two bf16 halves)."""
+def test_bf16_few_rows(hidden, ffn, heads, kv_heads, rows):
+    """bf16 weights over few rows, on both sides of the few-row form's ends
+    (15 rows, one round of blocks): 1e-4 of the row's magnitude (activations
+    as two bf16 halves)."""
     print(f"bf16 rows {rows} hidden {hidden} ffn {ffn}", flush=True)
-    cfg = synth.llama_config(2, hidden, 4, 2, ffn, 131, head_dim=32 if hidden < 512 else 64)
-    tensors = synth.make_tensors(cfg, 9, "bf16", std=0.05)
+    wide = hidden > 4000
+    cfg = synth.llama_config(1 if wide else 2, hidden, heads, kv_heads, ffn, 131, head_dim=hidden // heads)
+    tensors = synth.make_tensors(cfg, 9, "bf16", std=0.02 if wide else 0.05, fast=wide)
     ref = oracle.OracleModel(cfg, tensors)
     _rows_match(DecoderModel.from_bytes(cfg, st.dump(tensors), "bf16"), ref, 131, rows, 1e-4)
 
