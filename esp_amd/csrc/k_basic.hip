@@ -53,9 +53,9 @@ void launch_embed(Dt wt, const void *embed, const int32_t *ids, int M, int H, fl
 
 // ---------------------------------------------------------------- rmsnorm
 // burn-nn RmsNorm (built at layer.rs:27-33): y = x / sqrt(mean(x^2) + eps) * gamma.
-template <typename OT, bool SPLIT>
+template <bool SPLIT>
 __global__ void __launch_bounds__(256) rmsnorm_k(const float *x, const float *gamma, float eps,
-                                                 int H, OT *out, const int32_t *row_index) {
+                                                 int H, void *out, const int32_t *row_index) {
     __shared__ float red[16];
     int m = blockIdx.x;
     int src = row_index ? row_index[m] : m;
@@ -68,7 +68,7 @@ __global__ void __launch_bounds__(256) rmsnorm_k(const float *x, const float *ga
     for (int j = threadIdx.x; j < H; j += blockDim.x) {
         float y = (xr[j] / rms) * gamma[j];
         if (SPLIT) st_split((uint16_t *)out, plane, (size_t)m * H + j, y);
-        else st(out, (size_t)m * H + j, y);
+        else st((float *)out, (size_t)m * H + j, y);
     }
 }
 
@@ -187,8 +187,8 @@ __global__ void __launch_bounds__(NT) norm_block_k(NormArgs a) {
         }
     }
     // The sum of squares in an order that does not depend on the block's
-    // size: every wave adds the quads' sums itself, PLAIN and EMBED as lane l
-    // over quads l + 64 i (COMBINE too), RESID as four parts over quads 64 p + l + 256 i.
+    // size: every wave adds the quads' sums itself, lane l over quads l + 64 i
+    // (RESID: in four parts p, over quads 64 p + l + 256 i).
 #pragma unroll
     for (int i = 0; i < NQ; ++i)
         sq[tid + NT * i] = v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
@@ -241,7 +241,8 @@ bool resid_norm_ok(int H) { return H > 0 && H % 4 == 0 && H <= 8192; }
 
 void launch_rmsnorm(const float *x, const float *gamma, float eps, int M, int H, Dt out_dt,
                     void *out, const int32_t *row_index, hipStream_t s) {
-    if (resid_norm_ok(H) && out_dt != DT_BF16) {
+    if (out_dt != DT_SPLIT && out_dt != DT_F32) fail(ESP_BACKEND, "rmsnorm: f32 or split output only");
+    if (resid_norm_ok(H)) {
         NormArgs a{};
         a.x = const_cast<float *>(x);  // read only in this mode
         a.gamma = gamma;
@@ -254,12 +255,8 @@ void launch_rmsnorm(const float *x, const float *gamma, float eps, int M, int H,
         else norm_block<false, NB_PLAIN, float>(a, s);
         return;
     }
-    if (out_dt == DT_SPLIT)
-        rmsnorm_k<uint16_t, true><<<M, 256, 0, s>>>(x, gamma, eps, H, (uint16_t *)out, row_index);
-    else if (out_dt == DT_BF16)
-        rmsnorm_k<uint16_t, false><<<M, 256, 0, s>>>(x, gamma, eps, H, (uint16_t *)out, row_index);
-    else
-        rmsnorm_k<float, false><<<M, 256, 0, s>>>(x, gamma, eps, H, (float *)out, row_index);
+    if (out_dt == DT_SPLIT) rmsnorm_k<true><<<M, 256, 0, s>>>(x, gamma, eps, H, out, row_index);
+    else rmsnorm_k<false><<<M, 256, 0, s>>>(x, gamma, eps, H, out, row_index);
 }
 
 void launch_resid_norm(const float *ws, int splits, int M, int H, const float *bias, float *x,

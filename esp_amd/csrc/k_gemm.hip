@@ -14,9 +14,10 @@ void launch_gemm_packed(Dt wt, GemmEpi epi, const GemmArgs &a, hipStream_t s);
 
 bool gemm_takes_rows(Dt wt, const GemmArgs &a) { return gemm_mfma_ok(wt, a) && gemm_rows_ok(a); }
 
-// bf16 weights go to the bf16 matrix cores (activations split into bf16 hi +
-// lo), packed weights too, f32 weights to the f32 ones; K that is no multiple of 16 (bf16: 8) and
-// unaligned operands use the vector-ALU kernel.
+// bf16 and packed weights go to the bf16 matrix cores (activations split into
+// bf16 hi + lo), f32 weights to the f32 ones. The vector-ALU kernel takes what
+// they do not: f32 with K no multiple of 16, bf16 with K no multiple of 8 or
+// below 32, unaligned operands.
 void launch_gemm(Dt wt, GemmEpi epi, const GemmArgs &a, hipStream_t s) {
     if (a.defer_splits) *a.defer_splits = 0;
     if (a.M <= 0 || a.N <= 0) return;

@@ -18,8 +18,6 @@
 // rows gate/up 434 -> 208 (97 TFLOP/s), o and down 904 -> 77 on average,
 // q/k/v 379 -> 54; 8 rows gate/up ~1700 -> 32 (134 MB of weights, partly
 // from the memory-side cache).
-#include <utility>
-
 #include "common.hpp"
 #include "dev.hpp"
 #include "kernels_extra.hpp"
@@ -185,23 +183,25 @@ bool gemm_f32_ok(Dt wt, const GemmArgs &a) {
            a.grp_w_stride % 4 == 0 && al16(a.a) && al16(a.w) && (!a.w2 || al16(a.w2));
 }
 
-// Split count of a launch and its estimated time (us). `key_us` is the time
-// a CU spends on 16 keys of one tile divided by 16 (the matrix-core time of
-// the tile's blocks; measured, one tile per CU): `tiles * s` tiles of K / s
-// keys run in ceil(tiles s / cus) rounds, so splits pay where they even the
-// last round out, against the reduction launch (~4 us) and the partial sums
-// written and read once (~4 TB/s). Up to 32 rows the weight stream bounds the
-// launch instead and wants two blocks per CU. A split keeps at least 256 keys.
+// Whether `s` k splits, of at least 256 keys each, have room for their sums.
+static bool fg_split_fits(const GemmArgs &a, int NB, int s) {
+    return s <= 32 && a.K / s >= 256 && a.ws && (size_t)s * NB * a.M * a.N * 4 <= a.ws_bytes;
+}
+
+// Split count of a launch above 32 rows and its estimated time (us). `key_us`
+// is the time a CU spends on 16 keys of one tile divided by 16 (the
+// matrix-core time of the tile's blocks; measured, one tile per CU): `tiles *
+// s` tiles of K / s keys run in ceil(tiles s / cus) rounds, so splits pay
+// where they even the last round out, against the reduction launch (~4 us)
+// and the partial sums written and read once (~4 TB/s).
 static int fg_splits(const GemmArgs &a, int NB, long long tiles, double key_us, int cus, double *us) {
     int best = 1;
     double cost = 0;
-    for (int s = 1; s == 1 || (s <= 32 && a.K / s >= 256 && a.ws &&
-                               (size_t)s * NB * a.M * a.N * 4 <= a.ws_bytes); s *= 2) {
+    for (int s = 1; s == 1 || fg_split_fits(a, NB, s); s *= 2) {
         const double bytes = (double)s * NB * a.M * a.N * 8;
         const double c = (double)((tiles * s + cus - 1) / cus) * a.K / s * key_us +
                          (s > 1 ? 4.0 + bytes * 2.5e-7 : 0.0);
-        const bool fill = a.M <= 32 && s > 1 && tiles * (s / 2) < 2 * cus;
-        if (s == 1 || fill || (a.M > 32 && c < cost)) best = s, cost = c;
+        if (s == 1 || c < cost) best = s, cost = c;
     }
     *us = cost;
     return best;
@@ -250,8 +250,11 @@ template <int EPI> static void fg_dispatch(const GemmArgs &a, hipStream_t s) {
     constexpr double T64 = 0.0210, T128 = 0.0361, T256 = 0.0674;
     double u0, u1, u2;
     if (a.M <= 32) {
+        // the weight stream bounds these: splits until two blocks per CU
         constexpr int ST = NB == 1 ? 6 : 4;
-        const int sp = fg_splits(a, NB, fg_tiles<NB, 1, 1, 1, ST>(a), 0.0133 * NB, cus, &u0);
+        const long long tiles = fg_tiles<NB, 1, 1, 1, ST>(a);
+        int sp = 1;
+        while (tiles * sp < 2 * cus && fg_split_fits(a, NB, sp * 2)) sp *= 2;
         fg_launch<EPI, NB, 1, 1, 1, ST>(a, sp, s);
         return;
     }

@@ -10,9 +10,6 @@
 //
 // q4 nibbles are widened in the high half of a byte, as 16 q (exact in bf16
 // too), and the block's scale is divided by 16.
-#include <type_traits>
-#include <utility>
-
 #include "common.hpp"
 #include "dev.hpp"
 #include "kernels_extra.hpp"
@@ -58,11 +55,6 @@ __device__ __forceinline__ void pk_widen(const u32x4p_t &w, bf16x8p_t (&o)[2]) {
 __device__ __forceinline__ void pk_widen(const u32x2p_t &w, bf16x8p_t (&o)[2]) {
     o[0] = pk_bytes((w.x << 4) & 0xF0F0F0F0u, w.x & 0xF0F0F0F0u, true);
     o[1] = pk_bytes((w.y << 4) & 0xF0F0F0F0u, w.y & 0xF0F0F0F0u, true);
-}
-
-template <typename F, int... I>
-__device__ __forceinline__ void pk_static_for(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
 }
 
 template <int EPI, int NB>

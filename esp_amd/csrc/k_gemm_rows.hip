@@ -13,8 +13,6 @@
 // us (4.8 TB/s; before: 64-row tiles that met at every 32-key stage), o 10.1,
 // down 27, q/k/v 13.3; eight experts of 2048 x 7168 over 12 rows: gate/up 105
 // -> 81, down 90 -> 36 us (before: 128-row tiles, down unsplit).
-#include <type_traits>
-
 #include "common.hpp"
 #include "dev.hpp"
 #include "kernels_extra.hpp"

@@ -374,9 +374,8 @@ __global__ void __launch_bounds__(256) route_k(RouteArgs a) {
 }
 
 // Rows routed by a wave each read every logit once, so the router projection's
-// split sums are added there (a launch less per layer: two routed layers over
-// six rows 475 -> 468 us); the
-// other forms read a logit several times.
+// split sums are added there: a launch less per layer (two routed layers over
+// six rows 475 -> 468 us). The other forms read a logit several times.
 bool route_takes_splits(int M, int E) { return M <= 16 && E <= 64; }
 
 // More rows: the rows' top-k over the grid, one row per thread (one block
