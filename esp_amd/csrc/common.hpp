@@ -28,13 +28,14 @@ typedef uint16_t bf16_t;  // raw bf16 bits in host code
 
 // Element kinds. DT_SPLIT is an f32 activation matrix stored as two bf16
 // planes of the same shape, hi = bf16(x) then lo = bf16(x - hi), so matrix
-// cores can consume it exactly (R x C matrix: hi[r*C+c], lo[R*C + r*C+c]).
+// cores can consume it to 2^-17 (R x C matrix: hi[r*C+c], lo[R*C + r*C+c]).
+// DT_SPLIT3 adds a third plane, bf16(x - hi - lo): all 24 bits of x.
 // DT_Q8 / DT_Q4: packed projection weights, signed 8- or 4-bit integers
 // along K with one f32 scale per 32 inputs (values, then the scales).
 // DT_F16: IEEE binary16 (the K/V cache of the bf16 and packed formats).
-enum Dt { DT_F32 = 0, DT_BF16 = 1, DT_SPLIT = 2, DT_Q8 = 3, DT_Q4 = 4, DT_F16 = 5 };
+enum Dt { DT_F32 = 0, DT_BF16 = 1, DT_SPLIT = 2, DT_Q8 = 3, DT_Q4 = 4, DT_F16 = 5, DT_SPLIT3 = 6 };
 
-inline size_t dt_size(Dt d) { return d == DT_BF16 || d == DT_F16 ? 2 : 4; }
+inline size_t dt_size(Dt d) { return d == DT_BF16 || d == DT_F16 ? 2 : d == DT_SPLIT3 ? 6 : 4; }
 inline bool dt_packed(Dt d) { return d == DT_Q8 || d == DT_Q4; }
 // bytes of the packed values of n weights (n a multiple of 32)
 inline size_t packed_value_bytes(Dt d, size_t n) { return d == DT_Q8 ? n : n / 2; }
@@ -63,8 +64,8 @@ struct Rows {
 void launch_embed(Dt wt, const void *embed, const int32_t *ids, int M, int H, float *h,
                   hipStream_t s);
 
-// out[M,H] (dt out) = x / sqrt(mean(x^2)+eps) * gamma ; rows selected by
-// row_index (nullable = identity).
+// out[M,H] (DT_F32, DT_SPLIT or DT_SPLIT3) = x / sqrt(mean(x^2)+eps) * gamma ;
+// rows selected by row_index (nullable = identity).
 // x[m] += bias + sum_z ws[z][m] (the split-K partials of a RESIDUAL
 // projection, summed in split order as the GEMM reduction does), then
 // out = RMSNorm(x[m]) * gamma in out_dt (DT_SPLIT: hi/lo planes of M rows).
@@ -128,6 +129,8 @@ struct GemmArgs {
     // them, in split order); a launch without splits applies the epilogue and
     // stores 0.
     int *defer_splits;
+    // Packed weights, STORE only (nullable): the third plane of a DT_SPLIT3 A.
+    const void *a_lo2;
     // Packed weights (DT_Q8 / DT_Q4): the f32 block scales [N, K / 32] of w
     // and w2.
     const float *w_scale, *w2_scale;

@@ -36,11 +36,15 @@ template <> __device__ __forceinline__ void st<_Float16>(_Float16 *p, size_t i, 
     p[i] = (_Float16)v;
 }
 
-// Store x into a split (hi/lo bf16 planes) matrix; `plane` = elements per plane.
-__device__ __forceinline__ void st_split(uint16_t *base, size_t plane, size_t i, float x) {
-    uint16_t h = f2bf(x);
-    base[i] = h;
-    base[plane + i] = f2bf(x - bf2f(h));
+// Store x into a split matrix of P bf16 planes, each the rounding of what the
+// ones before it left; `plane` = elements per plane.
+template <int P = 2> __device__ __forceinline__ void st_split(uint16_t *base, size_t plane, size_t i, float x) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const uint16_t h = f2bf(x);
+        base[p * plane + i] = h;
+        x -= bf2f(h);
+    }
 }
 
 __device__ __forceinline__ float wave_sum(float v) {

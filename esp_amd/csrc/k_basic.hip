@@ -53,7 +53,8 @@ void launch_embed(Dt wt, const void *embed, const int32_t *ids, int M, int H, fl
 
 // ---------------------------------------------------------------- rmsnorm
 // burn-nn RmsNorm (built at layer.rs:27-33): y = x / sqrt(mean(x^2) + eps) * gamma.
-template <bool SPLIT>
+// P: 0 = f32 rows, 2 or 3 bf16 planes.
+template <int P>
 __global__ void __launch_bounds__(256) rmsnorm_k(const float *x, const float *gamma, float eps,
                                                  int H, void *out, const int32_t *row_index) {
     __shared__ float red[16];
@@ -67,7 +68,7 @@ __global__ void __launch_bounds__(256) rmsnorm_k(const float *x, const float *ga
     const size_t plane = (size_t)gridDim.x * H;
     for (int j = threadIdx.x; j < H; j += blockDim.x) {
         float y = (xr[j] / rms) * gamma[j];
-        if (SPLIT) st_split((uint16_t *)out, plane, (size_t)m * H + j, y);
+        if (P) st_split<P>((uint16_t *)out, plane, (size_t)m * H + j, y);
         else st((float *)out, (size_t)m * H + j, y);
     }
 }
@@ -96,7 +97,7 @@ struct NormArgs {
     const float *gamma;
     float eps;
     int M, H;
-    void *out;                 // f32 [M, H], or hi / lo planes of M rows
+    void *out;                 // f32 [M, H], or two or three bf16 planes of M rows
     const int32_t *row_index;  // PLAIN: nullable
     const float *ws, *bias;    // RESID: [splits][M][H], nullable [H]
     int splits;
@@ -145,7 +146,7 @@ __device__ __forceinline__ f32x4 combine4(const CombineArgs &c, int m, int j) {
     return out;
 }
 
-template <bool SPLIT, int NT, int NQ, int MODE, typename ET>
+template <int P, int NT, int NQ, int MODE, typename ET>
 __global__ void __launch_bounds__(NT) norm_block_k(NormArgs a) {
     __shared__ float sq[NT * NQ];
     const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, H = a.H;
@@ -211,37 +212,40 @@ __global__ void __launch_bounds__(NT) norm_block_k(NormArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = (v[i][e] / rms) * gv[i][e];
         const size_t o = (size_t)m * H + j;
-        if (SPLIT) {
-            uint16_t *out = (uint16_t *)a.out;
-            uint16_t hi[4], lo[4];
+        if (P) {
+            uint16_t *out = (uint16_t *)a.out + o;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                hi[e] = f2bf(y[e]);
-                lo[e] = f2bf(y[e] - bf2f(hi[e]));
+            for (int p = 0; p < P; ++p) {
+                uint16_t b[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    b[e] = f2bf(y[e]);
+                    y[e] -= bf2f(b[e]);
+                }
+                *(uint2 *)(out + p * MH) = make_uint2(b[0] | ((uint32_t)b[1] << 16), b[2] | ((uint32_t)b[3] << 16));
             }
-            *(uint2 *)(out + o) = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
-            *(uint2 *)(out + MH + o) = make_uint2(lo[0] | ((uint32_t)lo[1] << 16), lo[2] | ((uint32_t)lo[3] << 16));
         } else {
             *(f32x4 *)((float *)a.out + o) = f32x4{y[0], y[1], y[2], y[3]};
         }
     }
 }
 
-template <bool SPLIT, int MODE, typename ET> static void norm_block(const NormArgs &a, hipStream_t s) {
+template <int P, int MODE, typename ET> static void norm_block(const NormArgs &a, hipStream_t s) {
     const int q = a.H / 4;
-    if (q <= 64) norm_block_k<SPLIT, 64, 1, MODE, ET><<<a.M, 64, 0, s>>>(a);
-    else if (q <= 128) norm_block_k<SPLIT, 128, 1, MODE, ET><<<a.M, 128, 0, s>>>(a);
-    else if (q <= 256) norm_block_k<SPLIT, 256, 1, MODE, ET><<<a.M, 256, 0, s>>>(a);
-    else if (q <= 512) norm_block_k<SPLIT, 512, 1, MODE, ET><<<a.M, 512, 0, s>>>(a);
-    else if (q <= 1024) norm_block_k<SPLIT, 1024, 1, MODE, ET><<<a.M, 1024, 0, s>>>(a);
-    else norm_block_k<SPLIT, 1024, 2, MODE, ET><<<a.M, 1024, 0, s>>>(a);
+    if (q <= 64) norm_block_k<P, 64, 1, MODE, ET><<<a.M, 64, 0, s>>>(a);
+    else if (q <= 128) norm_block_k<P, 128, 1, MODE, ET><<<a.M, 128, 0, s>>>(a);
+    else if (q <= 256) norm_block_k<P, 256, 1, MODE, ET><<<a.M, 256, 0, s>>>(a);
+    else if (q <= 512) norm_block_k<P, 512, 1, MODE, ET><<<a.M, 512, 0, s>>>(a);
+    else if (q <= 1024) norm_block_k<P, 1024, 1, MODE, ET><<<a.M, 1024, 0, s>>>(a);
+    else norm_block_k<P, 1024, 2, MODE, ET><<<a.M, 1024, 0, s>>>(a);
 }
 
 bool resid_norm_ok(int H) { return H > 0 && H % 4 == 0 && H <= 8192; }
 
 void launch_rmsnorm(const float *x, const float *gamma, float eps, int M, int H, Dt out_dt,
                     void *out, const int32_t *row_index, hipStream_t s) {
-    if (out_dt != DT_SPLIT && out_dt != DT_F32) fail(ESP_BACKEND, "rmsnorm: f32 or split output only");
+    if (out_dt != DT_SPLIT && out_dt != DT_SPLIT3 && out_dt != DT_F32)
+        fail(ESP_BACKEND, "rmsnorm: f32 or split output only");
     if (resid_norm_ok(H)) {
         NormArgs a{};
         a.x = const_cast<float *>(x);  // read only in this mode
@@ -251,12 +255,14 @@ void launch_rmsnorm(const float *x, const float *gamma, float eps, int M, int H,
         a.H = H;
         a.out = out;
         a.row_index = row_index;
-        if (out_dt == DT_SPLIT) norm_block<true, NB_PLAIN, float>(a, s);
-        else norm_block<false, NB_PLAIN, float>(a, s);
+        if (out_dt == DT_SPLIT) norm_block<2, NB_PLAIN, float>(a, s);
+        else if (out_dt == DT_SPLIT3) norm_block<3, NB_PLAIN, float>(a, s);
+        else norm_block<0, NB_PLAIN, float>(a, s);
         return;
     }
-    if (out_dt == DT_SPLIT) rmsnorm_k<true><<<M, 256, 0, s>>>(x, gamma, eps, H, out, row_index);
-    else rmsnorm_k<false><<<M, 256, 0, s>>>(x, gamma, eps, H, out, row_index);
+    if (out_dt == DT_SPLIT) rmsnorm_k<2><<<M, 256, 0, s>>>(x, gamma, eps, H, out, row_index);
+    else if (out_dt == DT_SPLIT3) rmsnorm_k<3><<<M, 256, 0, s>>>(x, gamma, eps, H, out, row_index);
+    else rmsnorm_k<0><<<M, 256, 0, s>>>(x, gamma, eps, H, out, row_index);
 }
 
 void launch_resid_norm(const float *ws, int splits, int M, int H, const float *bias, float *x,
@@ -273,8 +279,8 @@ void launch_resid_norm(const float *ws, int splits, int M, int H, const float *b
     a.ws = ws;
     a.bias = bias;
     a.splits = splits;
-    if (out_dt == DT_SPLIT) norm_block<true, NB_RESID, float>(a, s);
-    else norm_block<false, NB_RESID, float>(a, s);
+    if (out_dt == DT_SPLIT) norm_block<2, NB_RESID, float>(a, s);
+    else norm_block<0, NB_RESID, float>(a, s);
 }
 
 void launch_combine_norm(const CombineArgs &c, const float *gamma, float eps, Dt out_dt, void *out, hipStream_t s) {
@@ -287,8 +293,8 @@ void launch_combine_norm(const CombineArgs &c, const float *gamma, float eps, Dt
     a.H = c.H;
     a.out = out;
     a.c = c;
-    if (out_dt == DT_SPLIT) norm_block<true, NB_COMBINE, float>(a, s);
-    else norm_block<false, NB_COMBINE, float>(a, s);
+    if (out_dt == DT_SPLIT) norm_block<2, NB_COMBINE, float>(a, s);
+    else norm_block<0, NB_COMBINE, float>(a, s);
 }
 
 bool embed_norm_ok(Dt wt, const void *embed, int H) {
@@ -306,10 +312,10 @@ void launch_embed_norm(Dt wt, const void *embed, const int32_t *ids, int M, int 
     a.out = out;
     a.embed = embed;
     a.ids = ids;
-    if (wt == DT_BF16 && out_dt == DT_SPLIT) norm_block<true, NB_EMBED, uint16_t>(a, s);
-    else if (wt == DT_BF16) norm_block<false, NB_EMBED, uint16_t>(a, s);
-    else if (out_dt == DT_SPLIT) norm_block<true, NB_EMBED, float>(a, s);
-    else norm_block<false, NB_EMBED, float>(a, s);
+    if (wt == DT_BF16 && out_dt == DT_SPLIT) norm_block<2, NB_EMBED, uint16_t>(a, s);
+    else if (wt == DT_BF16) norm_block<0, NB_EMBED, uint16_t>(a, s);
+    else if (out_dt == DT_SPLIT) norm_block<2, NB_EMBED, float>(a, s);
+    else norm_block<0, NB_EMBED, float>(a, s);
 }
 
 // ----------------------------------------------------------------- rope_kv

@@ -22,6 +22,7 @@ void launch_gemm(Dt wt, GemmEpi epi, const GemmArgs &a, hipStream_t s) {
     if (a.defer_splits) *a.defer_splits = 0;
     if (a.M <= 0 || a.N <= 0) return;
     if (dt_packed(wt)) launch_gemm_packed(wt, epi, a, s);
+    else if (a.a_lo2) fail(ESP_BACKEND, "GEMM: three activation planes outside the packed form");
     else if (gemm_takes_rows(wt, a)) launch_gemm_rows(epi, a, s);
     else if (a.a_rows) fail(ESP_BACKEND, "GEMM: row table outside the few-row form");
     else if (gemm_mfma_ok(wt, a)) launch_gemm_mfma(epi, a, a.ws, a.ws ? a.ws_bytes : 0, s);

@@ -2,11 +2,12 @@
 // cores, straight from the packed bytes:
 //   C[M,N] (f32) = A[M,K] . (q[N,K] * scale[N,K/32])^T
 // The integers are exact in bf16, so a 32-key block is multiplied as
-//   t = (a_hi + a_lo) . q      (v_mfma_f32_32x32x16_bf16, four per block)
+//   t = (a_hi + a_lo [+ a_lo2]) . q   (v_mfma_f32_32x32x16_bf16)
 // and joins the sum as acc += t * scale: two products per weight instead of
 // the three that a weight split into two bf16 halves needs, no dequantized
 // copy, and no rounding of q * scale. (t stays finite for |a| < 8e34.)
-// Activations arrive as bf16 hi / lo planes, as for bf16 weights.
+// Activations arrive as P bf16 planes: hi / lo, as for bf16 weights, or three
+// (the output head, whose activations stay whole).
 //
 // q4 nibbles are widened in the high half of a byte, as 16 q (exact in bf16
 // too), and the block's scale is divided by 16.
@@ -34,6 +35,10 @@ __device__ __forceinline__ int pk_swz(int r) { return (r >> 2) & 3; }
 constexpr int pk_vm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
 
 // sixteen keys of one weight row as loaded: 16 bytes (q8) or 8 bytes (q4)
+__device__ __forceinline__ const uint16_t *pk_plane(const GemmArgs &g, int p) {
+    return (const uint16_t *)(p == 0 ? g.a : p == 1 ? g.a_lo : g.a_lo2);
+}
+
 template <bool Q4> struct PkLoad { typedef u32x4p_t T; };
 template <> struct PkLoad<true> { typedef u32x2p_t T; };
 
@@ -101,8 +106,11 @@ __device__ __forceinline__ void pk_store(const GemmArgs &g, float *ws, int z, in
 // 61 -> 37 us (3.6 TB/s), q4 52 -> 28 us; dequantizing and multiplying the
 // bf16 halves took 250. Bound by the vector ALU's share of each block (widen,
 // scale, sum) and the latency of its chain.
-// activation keys resident in LDS
-template <int R> constexpr int ps_keys() { return R == 1 ? 512 : 256; }
+// Activation keys resident in LDS. Three planes of them (the output head) take
+// half the keys, so that a CU keeps as many blocks: a 128256 x 4096 head, us
+// with as many keys as two planes -> with half: q8 9 rows 205 -> 171, 64 rows
+// 593 -> 381, q4 9 rows 144 -> 120 (two planes: 161, 270, 107).
+template <int R, int P> constexpr int ps_keys() { return P == 3 ? (R == 1 ? 256 : 128) : R == 1 ? 512 : 256; }
 
 constexpr int PS_G = 4, PS_GK = 32 * PS_G;  // blocks and keys of a group
 
@@ -124,13 +132,13 @@ __device__ __forceinline__ void pk_transpose(uint32_t &x0, uint32_t &x1, uint32_
     pk_swap16(x2, x3);
 }
 
-template <int EPI, int NB, int R, bool Q4>
+template <int EPI, int NB, int R, bool Q4, int P>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1 ? 4 : 2)))
     gemm_pk_skinny_k(GemmArgs g, float *ws, int k_per_split) {
-    constexpr int G = PS_G, KEYS = PS_GK, NQ = Q4 ? 1 : 2, CK = ps_keys<R>(), GPC = CK / KEYS;
+    constexpr int G = PS_G, KEYS = PS_GK, NQ = Q4 ? 1 : 2, CK = ps_keys<R, P>(), GPC = CK / KEYS;
     constexpr int NC = 2 / NB;                       // 16-column groups per wave and matrix
     constexpr int BN = 64 * NC;                      // columns per block
-    constexpr int ROWS = 16 * R, APL = ROWS * PK_ROWB, AST = 2 * APL;  // a stage: hi plane, lo plane
+    constexpr int ROWS = 16 * R, APL = ROWS * PK_ROWB, AST = P * APL;  // a stage: its planes
     extern __shared__ __attribute__((aligned(16))) char lds_p[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int M = g.M, N = g.N, K = g.K;
@@ -165,11 +173,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1
     // (slot sl: row sl / 4, 16-byte chunk (sl % 4) ^ swz); rows past M repeat
     // the last, stages past the range are skipped
     auto bring_a = [&](int k0) {
-        const int n_ins = min(CK, kn - k0) / 32 * 2 * R;
+        const int n_ins = min(CK, kn - k0) / 32 * P * R;
         const int r16 = lane >> 2, kc = (lane & 3) ^ pk_swz(r16);
         for (int q = wave; q < n_ins; q += 4) {
-            const int st = q / (2 * R), p = q / R % 2, rb = q % R;
-            const uint16_t *src = (const uint16_t *)(p ? g.a_lo : g.a) + (size_t)min(rb * 16 + r16, M - 1) * K +
+            const int st = q / (P * R), p = q / R % P, rb = q % R;
+            const uint16_t *src = pk_plane(g, p) + (size_t)min(rb * 16 + r16, M - 1) * K +
                                   kbeg + k0 + st * 32 + kc * 8;
             __builtin_amdgcn_global_load_lds((gpptr_t)src, (lpptr_t)(lds_p + q * 1024), 16, 0, 0);
         }
@@ -206,13 +214,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1
             }
         }
         const char *base = lds_p + gi % GPC * G * AST;
-        bf16x8p_t fa[2][2][R];  // [stage parity][hi / lo]
-        auto read_a = [&](int st, bf16x8p_t (&o)[2][R]) {
+        bf16x8p_t fa[2][P][R];  // [stage parity][plane]
+        auto read_a = [&](int st, bf16x8p_t (&o)[P][R]) {
 #pragma unroll
             for (int i = 0; i < R; ++i) {
                 const int r = lane & 15, off = i * 1024 + r * PK_ROWB + (((lane >> 4) ^ pk_swz(r)) << 4);
-                o[0][i] = *(const bf16x8p_t *)(base + st * AST + off);
-                o[1][i] = *(const bf16x8p_t *)(base + st * AST + APL + off);
+#pragma unroll
+                for (int p = 0; p < P; ++p) o[p][i] = *(const bf16x8p_t *)(base + st * AST + p * APL + off);
             }
         };
         read_a(0, fa[0]);
@@ -222,7 +230,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1
             // left alone the compiler widens the whole group first and spills
             __builtin_amdgcn_sched_barrier(0);
             if (st + 1 < G) read_a(st + 1, fa[(st + 1) & 1]);
-            const bf16x8p_t (&fh)[R] = fa[st & 1][0], (&fl)[R] = fa[st & 1][1];
+            const bf16x8p_t (&fs)[P][R] = fa[st & 1];
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 bf16x8p_t f;
@@ -236,8 +244,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1
                 const float s = Q4 ? w.s[u][st] * 0.0625f : w.s[u][st];
 #pragma unroll
                 for (int i = 0; i < R; ++i) {
-                    f32x4p_t t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh[i], f, (f32x4p_t)(0.f), 0, 0, 0);
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl[i], f, t, 0, 0, 0);
+                    f32x4p_t t = (f32x4p_t)(0.f);
+#pragma unroll
+                    for (int p = 0; p < P; ++p) t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fs[p][i], f, t, 0, 0, 0);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) acc[u][i][e] = fmaf(t[e], s, acc[u][i][e]);
                 }
@@ -283,13 +292,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1
 // took 1500; 1100 rows, four projections of a layer: 2.25 -> 1.15 ms.
 constexpr int PT_BM = 128, PT_BR = 256;
 constexpr int PT_A = PT_BM * PK_ROWB;  // one plane of a stage
-constexpr int PT_STAGE = 2 * PT_A + PT_BR * PK_ROWB + PT_BR * 4;
-constexpr size_t PT_LDS = 2 * PT_STAGE;
+template <int P> constexpr int pt_stage() { return P * PT_A + PT_BR * PK_ROWB + PT_BR * 4; }
+template <int P> constexpr size_t pt_lds() { return 2 * pt_stage<P>(); }
 
-template <int EPI, int NB, bool Q4>
-__global__ void __launch_bounds__(256, 2) gemm_pk_tile_k(GemmArgs g, float *ws, int k_per_split, int mt, int nt) {
+// three planes: one block per CU (82 KB of LDS; a 128256 x 4096 q8 head of 100
+// rows 361 -> 540 us against two planes, 3375 dequantized in f32)
+template <int EPI, int NB, bool Q4, int P>
+__global__ void __launch_bounds__(256, P == 2 ? 2 : 1) gemm_pk_tile_k(GemmArgs g, float *ws, int k_per_split, int mt, int nt) {
     typedef typename PkLoad<Q4>::T W;
     constexpr int BN = PT_BR / NB, NJ = BN / 64;  // 32-column blocks per wave and matrix
+    constexpr int PT_STAGE = pt_stage<P>();
     extern __shared__ __attribute__((aligned(16))) char lds_p[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int wm = wave >> 1, wn = wave & 1;
@@ -307,13 +319,13 @@ __global__ void __launch_bounds__(256, 2) gemm_pk_tile_k(GemmArgs g, float *ws, 
 
     // activation rows: 8 instructions of 16 rows per plane, two per wave;
     // rows past M repeat the last
-    const uint16_t *asrc[2][2];
+    const uint16_t *asrc[P][2];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
         const int sl = (wave * 2 + q) * 64 + lane, r = sl >> 2, kc = (sl & 3) ^ pk_swz(r);
         const size_t off = (size_t)min(m0 + r, M - 1) * K + kbeg + kc * 8;
-        asrc[0][q] = (const uint16_t *)g.a + off;
-        asrc[1][q] = (const uint16_t *)g.a_lo + off;
+#pragma unroll
+        for (int p = 0; p < P; ++p) asrc[p][q] = pk_plane(g, p) + off;
     }
     // packed values: thread = (weight row tid / 2 + 128 i, keys 16 (tid & 1)
     // .. + 16); scale: weight row tid
@@ -332,7 +344,7 @@ __global__ void __launch_bounds__(256, 2) gemm_pk_tile_k(GemmArgs g, float *ws, 
     auto issue_a = [&](int kt) {
         char *base = lds_p + (kt & 1) * PT_STAGE;
 #pragma unroll
-        for (int p = 0; p < 2; ++p)
+        for (int p = 0; p < P; ++p)
 #pragma unroll
             for (int q = 0; q < 2; ++q)
                 __builtin_amdgcn_global_load_lds((gpptr_t)(asrc[p][q] + kt * 32),
@@ -344,7 +356,7 @@ __global__ void __launch_bounds__(256, 2) gemm_pk_tile_k(GemmArgs g, float *ws, 
         sr = ssrc[kt];
     };
     auto put_w = [&](int kt) {  // registers -> LDS, widened
-        char *bb = lds_p + (kt & 1) * PT_STAGE + 2 * PT_A;
+        char *bb = lds_p + (kt & 1) * PT_STAGE + P * PT_A;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int r = (tid >> 1) + 128 * i;
@@ -385,19 +397,19 @@ __global__ void __launch_bounds__(256, 2) gemm_pk_tile_k(GemmArgs g, float *ws, 
             if (kt + 2 < KT) issue_w(kt + 2);
         }
         __builtin_amdgcn_sched_barrier(0);
-        const char *ah = lds_p + (kt & 1) * PT_STAGE, *al = ah + PT_A, *bb = al + PT_A;
+        const char *ab = lds_p + (kt & 1) * PT_STAGE, *bb = ab + P * PT_A;
         const float *sc = (const float *)(bb + PT_BR * PK_ROWB);
-        bf16x8p_t fh[2][2], fl[2][2];
+        bf16x8p_t fs[P][2][2];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int c = 2 * ks + (lane >> 5), r = wm * 64 + i * 32 + (lane & 31);
                 const int off = r * PK_ROWB + ((c ^ pk_swz(r)) << 4);
-                fh[ks][i] = *(const bf16x8p_t *)(ah + off);
-                fl[ks][i] = *(const bf16x8p_t *)(al + off);
+#pragma unroll
+                for (int p = 0; p < P; ++p) fs[p][ks][i] = *(const bf16x8p_t *)(ab + p * PT_A + off);
             }
-        // Units of one 32 x 32 block: a unit's four products are issued with
+        // Units of one 32 x 32 block: a unit's 2 P products are issued with
         // the previous unit's sixteen sums between them, so the vector ALU
         // works in the shadow of the matrix core, and two product blocks are
         // live at a time.
@@ -425,10 +437,10 @@ __global__ void __launch_bounds__(256, 2) gemm_pk_tile_k(GemmArgs g, float *ws, 
             __builtin_amdgcn_sched_barrier(0);
             f32x16p_t x = (f32x16p_t)(0.f);
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fh[ks][i], f[jb & 1][ks], x, 0, 0, 0);
-                x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fl[ks][i], f[jb & 1][ks], x, 0, 0, 0);
-            }
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+                    x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fs[p][ks][i], f[jb & 1][ks], x, 0, 0, 0);
             if (u > 0) sums(u - 1);
             t[u & 1] = x;
             if (i == 1 && jb + 1 < CB) read_w(jb + 1, f[(jb + 1) & 1], sv[(jb + 1) & 1]);
@@ -477,13 +489,13 @@ static void pk_finish(GemmEpi epi, const GemmArgs &a, int splits, hipStream_t s)
     else launch_gemm_reduce(epi, a, a.ws, splits, s);
 }
 
-template <int EPI, int NB, int R, bool Q4> static void pk_skinny(const GemmArgs &a, hipStream_t s) {
+template <int EPI, int NB, int R, bool Q4, int P> static void pk_skinny(const GemmArgs &a, hipStream_t s) {
     constexpr int KU = PS_GK, BN = 128 / NB;
-    constexpr size_t LDSB = (size_t)ps_keys<R>() * 16 * R * 4;
+    constexpr size_t LDSB = (size_t)ps_keys<R, P>() * 16 * R * 2 * P;
     static bool attr = false;
     if (!attr) {
-        for (const void *k : {reinterpret_cast<const void *>(gemm_pk_skinny_k<EPI, NB, R, Q4>),
-                              reinterpret_cast<const void *>(gemm_pk_skinny_k<PK_PARTIAL, NB, R, Q4>)})
+        for (const void *k : {reinterpret_cast<const void *>(gemm_pk_skinny_k<EPI, NB, R, Q4, P>),
+                              reinterpret_cast<const void *>(gemm_pk_skinny_k<PK_PARTIAL, NB, R, Q4, P>)})
             ESP_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDSB));
         attr = true;
     }
@@ -495,19 +507,19 @@ template <int EPI, int NB, int R, bool Q4> static void pk_skinny(const GemmArgs 
     const int kps = ((a.K + splits - 1) / splits + KU - 1) / KU * KU;
     splits = (a.K + kps - 1) / kps;
     if (splits == 1) {
-        gemm_pk_skinny_k<EPI, NB, R, Q4><<<dim3(gx), 256, LDSB, s>>>(a, nullptr, a.K);
+        gemm_pk_skinny_k<EPI, NB, R, Q4, P><<<dim3(gx), 256, LDSB, s>>>(a, nullptr, a.K);
         return;
     }
-    gemm_pk_skinny_k<PK_PARTIAL, NB, R, Q4><<<dim3(gx, 1, splits), 256, LDSB, s>>>(a, a.ws, kps);
+    gemm_pk_skinny_k<PK_PARTIAL, NB, R, Q4, P><<<dim3(gx, 1, splits), 256, LDSB, s>>>(a, a.ws, kps);
     pk_finish((GemmEpi)EPI, a, splits, s);
 }
 
-template <int EPI, int NB, bool Q4> static void pk_tile(GemmArgs a, hipStream_t s) {
+template <int EPI, int NB, bool Q4, int P> static void pk_tile(GemmArgs a, hipStream_t s) {
     static bool attr = false;
     if (!attr) {
-        for (const void *k : {reinterpret_cast<const void *>(gemm_pk_tile_k<EPI, NB, Q4>),
-                              reinterpret_cast<const void *>(gemm_pk_tile_k<PK_PARTIAL, NB, Q4>)})
-            ESP_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PT_LDS));
+        for (const void *k : {reinterpret_cast<const void *>(gemm_pk_tile_k<EPI, NB, Q4, P>),
+                              reinterpret_cast<const void *>(gemm_pk_tile_k<PK_PARTIAL, NB, Q4, P>)})
+            ESP_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pt_lds<P>()));
         attr = true;
     }
     constexpr int BN = PT_BR / NB;
@@ -532,29 +544,30 @@ template <int EPI, int NB, bool Q4> static void pk_tile(GemmArgs a, hipStream_t 
     const int kps = ((a.K + splits - 1) / splits + 31) / 32 * 32;
     splits = (a.K + kps - 1) / kps;
     if (splits == 1) {
-        gemm_pk_tile_k<EPI, NB, Q4><<<dim3(blocks), 256, PT_LDS, s>>>(a, nullptr, a.K, mt, nt);
+        gemm_pk_tile_k<EPI, NB, Q4, P><<<dim3(blocks), 256, pt_lds<P>(), s>>>(a, nullptr, a.K, mt, nt);
         return;
     }
-    gemm_pk_tile_k<PK_PARTIAL, NB, Q4><<<dim3(blocks, 1, splits), 256, PT_LDS, s>>>(a, a.ws, kps, mt, nt);
+    gemm_pk_tile_k<PK_PARTIAL, NB, Q4, P><<<dim3(blocks, 1, splits), 256, pt_lds<P>(), s>>>(a, a.ws, kps, mt, nt);
     pk_finish((GemmEpi)EPI, a, splits, s);
 }
 
-template <int EPI, bool Q4> static void pk_dispatch(const GemmArgs &a, hipStream_t s) {
+template <int EPI, bool Q4, int P = 2> static void pk_dispatch(const GemmArgs &a, hipStream_t s) {
     constexpr int NB = EPI == GEMM_SWIGLU ? 2 : 1;
     const bool line = a.K % PS_GK == 0;  // whole groups of every weight row
-    if (a.M <= 16 && line) pk_skinny<EPI, NB, 1, Q4>(a, s);
-    else if (a.M <= 32 && line) pk_skinny<EPI, NB, 2, Q4>(a, s);
-    else if (a.M <= 64 && line) pk_skinny<EPI, NB, 4, Q4>(a, s);
-    else pk_tile<EPI, NB, Q4>(a, s);
+    if (a.M <= 16 && line) pk_skinny<EPI, NB, 1, Q4, P>(a, s);
+    else if (a.M <= 32 && line) pk_skinny<EPI, NB, 2, Q4, P>(a, s);
+    else if (a.M <= 64 && line) pk_skinny<EPI, NB, 4, Q4, P>(a, s);
+    else pk_tile<EPI, NB, Q4, P>(a, s);
 }
 
 void launch_gemm_packed(Dt wt, GemmEpi epi, const GemmArgs &a, hipStream_t s) {
     auto al16 = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
     if (!a.a_lo || !a.w_scale || a.K % 32 || a.grp_offs || !al16(a.a) || !al16(a.a_lo) || !al16(a.w) ||
-        (epi == GEMM_SWIGLU && (!a.w2_scale || !al16(a.w2))))
+        (epi == GEMM_SWIGLU && (!a.w2_scale || !al16(a.w2))) || (a.a_lo2 && (epi != GEMM_STORE || !al16(a.a_lo2))))
         fail(ESP_BACKEND, "packed GEMM: operands outside the block-32 form");
     const bool q4 = wt == DT_Q4;
-    if (epi == GEMM_STORE) q4 ? pk_dispatch<GEMM_STORE, true>(a, s) : pk_dispatch<GEMM_STORE, false>(a, s);
+    if (a.a_lo2) q4 ? pk_dispatch<GEMM_STORE, true, 3>(a, s) : pk_dispatch<GEMM_STORE, false, 3>(a, s);
+    else if (epi == GEMM_STORE) q4 ? pk_dispatch<GEMM_STORE, true>(a, s) : pk_dispatch<GEMM_STORE, false>(a, s);
     else if (epi == GEMM_RESIDUAL) q4 ? pk_dispatch<GEMM_RESIDUAL, true>(a, s) : pk_dispatch<GEMM_RESIDUAL, false>(a, s);
     else q4 ? pk_dispatch<GEMM_SWIGLU, true>(a, s) : pk_dispatch<GEMM_SWIGLU, false>(a, s);
 }

@@ -805,7 +805,7 @@ static int32_t *xcd_err_word(Kv &kv) { return kv.tickets.as<int32_t>() + kXcdErr
 
 // lo plane of a split activation buffer holding rows x cols (nullptr for f32)
 static void *lo_plane(Dt act, const DevMem &b, int rows, int cols) {
-    return act == DT_SPLIT ? (void *)((uint16_t *)b.p + (size_t)rows * cols) : nullptr;
+    return act == DT_SPLIT || act == DT_SPLIT3 ? (void *)((uint16_t *)b.p + (size_t)rows * cols) : nullptr;
 }
 
 // element type of LoRA B rows (packed formats carry no LoRA)
@@ -1416,7 +1416,7 @@ static void ensure_scratch(Model &m, Kv &kv, int Mc, int n_seqs) {
     if (qkv_rows <= 0) fail(ESP_BACKEND, "layer geometry missing: no fused q/k/v rows");
     int fmax = std::max(m.F, std::max(m.Fe, m.Fs));
     kv.h.ensure((size_t)Mc * H * 4);
-    kv.xn.ensure((size_t)Mc * H * 4);
+    kv.xn.ensure(std::max((size_t)Mc * 4, (size_t)n_seqs * (dt_packed(m.ht) ? 6 : 4)) * H);  // layers; head
     kv.qkv.ensure((size_t)Mc * qkv_rows * 4);
     kv.q.ensure((size_t)Mc * m.qw * 4);
     kv.attn.ensure((size_t)Mc * m.qw * 4);
@@ -1518,7 +1518,9 @@ static void run_head(Model &m, Kv &kv, int n_seqs, const float *h_src, const int
         launch_gemv(m.ht, GEMV_STORE, g, s);
         return;
     }
-    const Dt act = m.ht == DT_F32 ? DT_F32 : DT_SPLIT;
+    // a packed head keeps all 24 bits of the final norm, as the one-sequence
+    // head does (two planes: 2.4e-6 of the logits at K 4096, three 2e-7)
+    const Dt act = m.ht == DT_F32 ? DT_F32 : dt_packed(m.ht) ? DT_SPLIT3 : DT_SPLIT;
     {
         Prof p("rmsnorm", s);
         launch_rmsnorm(h_src, m.final_norm, m.cfg.rms_norm_eps, n_seqs, m.H, act, kv.xn.p, row_index, s);
@@ -1528,6 +1530,7 @@ static void run_head(Model &m, Kv &kv, int n_seqs, const float *h_src, const int
     g.ws_bytes = kv.gemm_ws.bytes;
     g.a = kv.xn.p;
     g.a_lo = lo_plane(act, kv.xn, n_seqs, m.H);
+    if (act == DT_SPLIT3) g.a_lo2 = kv.xn.as<uint16_t>() + (size_t)2 * n_seqs * m.H;
     g.w = m.head;
     g.w_scale = m.head_s;
     g.c = kv.logits.p;

@@ -55,6 +55,34 @@ def test_packed_rows(bits, hidden, ffn, rows):
     _rows_match(DecoderModel.from_bytes(cfg, st.dump(art), f"q{bits}-block32"), ref, 131, rows, 1e-4)
 
 
+# every form of the packed head: 16, 32 and 64 resident rows, tiles above; a K
+# without whole 128-key groups (tiles only)
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("hidden,rows", [(2048, 2), (2048, 17), (2048, 64), (2048, 131), (1088, 5)])
+def test_packed_head_keeps_f32_activations(bits, hidden, rows):
+    """The packed head of several sequences against 64 bits, on hidden states
+    that are the embeddings (zero output projections): 6e-7 of the logits,
+    which f32 operands and sums over K / 32 blocks keep (about 2e-7) and
+    activations of two bf16 halves do not (2.3e-6 at any K)."""
+    print(f"packed head q{bits} K {hidden} rows {rows}", flush=True)
+    cfg = synth.llama_config(1, hidden, 2, 2, 64, 515, head_dim=32)
+    tensors = synth.make_tensors(cfg, 9, "f32", std=0.05)
+    for name in ("self_attn.o_proj", "mlp.down_proj"):
+        tensors[f"model.layers.0.{name}.weight"][0][:] = 0
+    art = quant.convert_artifact(tensors, bits)
+    deq = quant.dequantized_model(art, {n: a.shape for n, (a, _) in tensors.items()}, bits)
+    model = DecoderModel.from_bytes(cfg, st.dump(art), f"q{bits}-block32")
+    ids = synth.uniform_ids(rows, rows, 515)
+    x = np.asarray(deq["model.embed_tokens.weight"][0], np.float64)[ids]
+    x = x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-5) * np.asarray(deq["model.norm.weight"][0], np.float64)
+    want = x @ np.asarray(deq["lm_head.weight"][0], np.float64).T
+    got = model.forward_batch(model.new_cache(rows, 4), list(range(rows)), [[t] for t in ids])
+    one = model.try_forward_cached_last([ids[0]], model.new_cache(1, 4))
+    rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert rel <= 6e-7, rel
+    assert np.linalg.norm(one - want[0]) <= 6e-7 * np.linalg.norm(want[0])
+
+
 @pytest.mark.parametrize("kv", ["f32", "f16"])
 @pytest.mark.parametrize("lens", [(16, 128, 129), (257, 16, 31, 400), (1100, 20), (2050, 2049, 40)])
 def test_prompt_blocks_in_one_launch(kv, lens):
