@@ -5,7 +5,9 @@
 //   t = (a_hi + a_lo [+ a_lo2]) . q   (v_mfma_f32_32x32x16_bf16)
 // and joins the sum as acc += t * scale: two products per weight instead of
 // the three that a weight split into two bf16 halves needs, no dequantized
-// copy, and no rounding of q * scale. (t stays finite for |a| < 8e34.)
+// copy, and no rounding of q * scale. t overflows from |a| = 8e34 on, where
+// a . (q * scale) need not: a block whose sums are not all finite computes its
+// outputs again with the scale inside (pk_plain).
 // Activations arrive as P bf16 planes: hi / lo, as for bf16 weights, or three
 // (the output head, whose activations stay whole).
 //
@@ -85,6 +87,36 @@ __device__ __forceinline__ void pk_store(const GemmArgs &g, float *ws, int z, in
     float *c = (float *)g.c + ci;
     const float y = g.bias ? v[0] + bias : v[0];
     *c = EPI == GEMM_RESIDUAL ? *c + y : y;
+}
+
+// Whether a launch can meet activations above 8e34: o_proj and down_proj (one
+// matrix, two planes) can; what reads a norm's output stays below sqrt(H) times
+// an f16 weight.
+template <int EPI, int NB, int P> constexpr bool pk_may_overflow() {
+    return NB == 1 && P == 2 && (EPI == GEMM_RESIDUAL || EPI == PK_PARTIAL);
+}
+__device__ __forceinline__ bool pk_finite(float x) { return fabsf(x) < INFINITY; }
+
+// The block's outputs (rows [m0, m0 + rows), columns [n0, n0 + cols), keys [k0,
+// k0 + kn)) as plain sums of a * (q * scale), for a block of 256 threads. An
+// output that is not finite here either ends its own sum.
+template <int EPI, bool Q4>
+__device__ void pk_plain(const GemmArgs &g, float *ws, int z, int m0, int rows, int n0, int cols, int k0, int kn) {
+    rows = min(rows, g.M - m0);
+    cols = min(cols, g.N - n0);
+    for (int i = threadIdx.x; i < rows * cols; i += 256) {
+        const int row = m0 + i / cols, col = n0 + i % cols;
+        const uint16_t *ah = (const uint16_t *)g.a + (size_t)row * g.K, *al = (const uint16_t *)g.a_lo + (size_t)row * g.K;
+        float acc = 0.f;
+        for (int k = k0; k < k0 + kn && pk_finite(acc); ++k) {
+            const size_t e = (size_t)col * g.K + k;
+            const int q = Q4 ? (int)((unsigned)((const uint8_t *)g.w)[e / 2] << (28 - 4 * (int)(e & 1))) >> 28
+                             : ((const int8_t *)g.w)[e];
+            acc = fmaf(bf2f(ah[k]) + bf2f(al[k]), (float)q * g.w_scale[e / 32], acc);
+        }
+        const float v[1] = {acc};
+        pk_store<EPI, 1>(g, ws, z, row, col, v, EPI != PK_PARTIAL && g.bias ? g.bias[col] : 0.f);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -258,6 +290,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1
     for (int gi = 0; gi < NG; gi += 2) {
         group(w0, w1, gi);
         if (gi + 1 < NG) group(w1, w0, gi + 1);
+    }
+    if constexpr (pk_may_overflow<EPI, NB, P>()) {
+        bool bad = false;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bad |= !pk_finite(acc[u][i][e]);
+        if (__syncthreads_or(bad)) {
+            pk_plain<EPI, Q4>(g, ws, blockIdx.z, 0, M, n0, BN, kbeg, kn);
+            return;
+        }
     }
 
     // a 16 x 16 block: column lane & 15, rows 4 (lane >> 4) + e
@@ -453,6 +498,19 @@ __global__ void __launch_bounds__(256, P == 2 ? 2 : 1) gemm_pk_tile_k(GemmArgs g
             }
         }
         sums(2 * CB - 1);
+    }
+    if constexpr (pk_may_overflow<EPI, NB, P>()) {
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) bad |= !pk_finite(acc[0][i][j][e]);
+        if (__syncthreads_or(bad)) {
+            pk_plain<EPI, Q4>(g, ws, blockIdx.z, m0, PT_BM, n0, BN, kbeg, KT * 32);
+            return;
+        }
     }
 
 #pragma unroll

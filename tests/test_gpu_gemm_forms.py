@@ -83,6 +83,25 @@ def test_packed_head_keeps_f32_activations(bits, hidden, rows):
     assert np.linalg.norm(one - want[0]) <= 6e-7 * np.linalg.norm(want[0])
 
 
+# 16, 32 and 64 resident rows and tiles, with k splits (hidden 512, ffn 1408)
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("rows", [2, 17, 40, 70])
+def test_packed_products_keep_the_f32_range(bits, rows):
+    """Values and gated units around 5e36 (up to 6e37) into o_proj and down_proj
+    weights around 5e-37: 32 integers times them leave the range of f32, times
+    the block's scale they do not. The outputs are the dequantized weights' own
+    (1e-4 of the row's magnitude, as in range)."""
+    print(f"packed range q{bits} rows {rows}", flush=True)
+    cfg = synth.llama_config(1, 512, 8, 4, 1408, 131, head_dim=64)
+    tensors = synth.make_tensors(cfg, 9, "f32", std=0.05)
+    for name, s in (("self_attn.v_proj", 4e36), ("self_attn.o_proj", 1e-35), ("mlp.up_proj", 4e36),
+                    ("mlp.down_proj", 1e-35)):
+        tensors[f"model.layers.0.{name}.weight"][0][:] *= np.float32(s)
+    art = quant.convert_artifact(tensors, bits)
+    ref = oracle.OracleModel(cfg, quant.dequantized_model(art, {n: a.shape for n, (a, _) in tensors.items()}, bits))
+    _rows_match(DecoderModel.from_bytes(cfg, st.dump(art), f"q{bits}-block32"), ref, 131, rows, 1e-4)
+
+
 @pytest.mark.parametrize("kv", ["f32", "f16"])
 @pytest.mark.parametrize("lens", [(16, 128, 129), (257, 16, 31, 400), (1100, 20), (2050, 2049, 40)])
 def test_prompt_blocks_in_one_launch(kv, lens):
