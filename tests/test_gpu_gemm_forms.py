@@ -38,8 +38,46 @@ def test_f32_rows(hidden, ffn, rows):
     _rows_match(DecoderModel.from_bytes(cfg, blob, "f32"), oracle.OracleModel(cfg, tensors), 131, rows, 1e-4)
 
 
-# K 96 (no skinny form: K % 128), 256 (skinny at both row counts), 640 =
-# K % 128 only, and k splits with a ragged last one at 1408
+# 128-row tiles: gate/up and the head (K 64, 116 rows in the last tile), and
+# down_proj in eight k splits (640 keys, one row in the last tile)
+@pytest.mark.parametrize("hidden,ffn,vocab,rows", [(64, 4096, 8192, 500), (1280, 5120, 131, 257)])
+def test_f32_128_row_tiles(hidden, ffn, vocab, rows):
+    """The f32 tile of 128 x 128, which wide products of many rows take: 1e-4 of
+    the row's magnitude, as above."""
+    print(f"f32 128-row tiles hidden {hidden} ffn {ffn} rows {rows}", flush=True)
+    cfg, tensors, blob, _ = synth.tiny_llama_case(seed=6, layers=1, hidden=hidden, heads=hidden // 16,
+                                                  kv_heads=hidden // 16, ffn=ffn, vocab=vocab, prompt_len=2)
+    _rows_match(DecoderModel.from_bytes(cfg, blob, "f32"), oracle.OracleModel(cfg, tensors), vocab, rows, 1e-4)
+
+
+# q/k/v in four k splits, which the rotary pass adds up (head_dim 64 and 128)
+@pytest.mark.parametrize("arch,head_dim", [("llama", 64), ("qwen2", 128), ("qwen2", 64), ("qwen3", 128)])
+@pytest.mark.parametrize("lens", [(2, 5), (9, 17, 14), (60, 70)])
+def test_f32_split_qkv_rows(arch, head_dim, lens):
+    """f32 models whose q/k/v sums reach the rotary pass as k splits, with the
+    q/k/v bias (qwen2) and the per-head q/k norm (qwen3): several sequences'
+    blocks, so that every query reads other rows' keys; 1e-4 of the row's
+    magnitude."""
+    print(f"f32 split q/k/v {arch} hd {head_dim} blocks {lens}", flush=True)
+    names = {"llama": "LlamaForCausalLM", "qwen2": "Qwen2ForCausalLM", "qwen3": "Qwen3ForCausalLM"}
+    cfg = synth.llama_config(2, 1024, 1024 // head_dim, 4, 1024, 131, head_dim=head_dim,
+                             extra={"architectures": [names[arch]], "model_type": arch})
+    assert cfg.qkv_bias() == (arch == "qwen2") and cfg.qk_norm() == (arch == "qwen3")
+    tensors = synth.make_tensors(cfg, 4, "f32", std=0.05, bias_std=0.5)
+    for name in tensors:  # weights of the per-head norms, which are 1 otherwise
+        if name.endswith(("q_norm.weight", "k_norm.weight")):
+            tensors[name][0][:] = 1 + synth.normal(synth.tensor_seed(4, name), head_dim, 0.3)
+    model, ref = DecoderModel.from_bytes(cfg, st.dump(tensors), "f32"), oracle.OracleModel(cfg, tensors)
+    blocks = [synth.uniform_ids(3 + i, n, 131) for i, n in enumerate(lens)]
+    got = model.forward_batch(model.new_cache(len(lens), max(lens)), list(range(len(lens))), blocks)
+    for r, b in enumerate(blocks):
+        want = ref.forward_last(ref.new_cache(), b)
+        err = float(np.abs(got[r] - want).max())
+        assert err <= 1e-4 * float(np.abs(want).max()), f"sequence {r} of {lens}: {err}"
+
+
+# K 128 (one group of keys), 192 (no whole groups: tiles at any row count), 256,
+# 512, 640, and 1408 in ragged k splits
 @pytest.mark.parametrize("bits", [8, 4])
 @pytest.mark.parametrize("hidden,ffn", [(128, 192), (256, 640), (512, 1408)])
 @pytest.mark.parametrize("rows", [2, 31, 32, 33, 64, 65, 129, 300])
@@ -55,24 +93,41 @@ def test_packed_rows(bits, hidden, ffn, rows):
     _rows_match(DecoderModel.from_bytes(cfg, st.dump(art), f"q{bits}-block32"), ref, 131, rows, 1e-4)
 
 
-# every form of the packed head: 16, 32 and 64 resident rows, tiles above; a K
-# without whole 128-key groups (tiles only)
+# gate/up of 16384 columns fill two blocks per CU with two k splits, of 640 keys:
+# the resident 512 (16 rows) or 256 are refilled, the last time in part
 @pytest.mark.parametrize("bits", [8, 4])
-@pytest.mark.parametrize("hidden,rows", [(2048, 2), (2048, 17), (2048, 64), (2048, 131), (1088, 5)])
-def test_packed_head_keeps_f32_activations(bits, hidden, rows):
+@pytest.mark.parametrize("rows", [2, 16, 32, 64])
+def test_packed_rows_refill_their_activations(bits, rows):
+    """Packed products whose k range is longer than the resident activations:
+    1e-4 of the row's magnitude."""
+    print(f"q{bits} refill rows {rows}", flush=True)
+    cfg = synth.llama_config(1, 1280, 10, 2, 16384, 131, head_dim=128)
+    tensors = synth.make_tensors(cfg, 9, "f32", std=0.02, fast=True)
+    art = quant.convert_artifact(tensors, bits)
+    ref = oracle.OracleModel(cfg, quant.dequantized_model(art, {n: a.shape for n, (a, _) in tensors.items()}, bits))
+    _rows_match(DecoderModel.from_bytes(cfg, st.dump(art), f"q{bits}-block32"), ref, 131, rows, 1e-4)
+
+
+# every form of the packed head: 16, 32 and 64 resident rows, tiles above; a K
+# without whole 128-key groups (tiles only); 65500 columns fill the chip without
+# k splits, so that the 256 (9 rows) or 128 resident keys are refilled
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("hidden,rows,vocab", [(2048, 2, 515), (2048, 17, 515), (2048, 64, 515), (2048, 131, 515),
+                                               (1088, 5, 515), (640, 9, 65500), (640, 20, 65500)])
+def test_packed_head_keeps_f32_activations(bits, hidden, rows, vocab):
     """The packed head of several sequences against 64 bits, on hidden states
     that are the embeddings (zero output projections): 6e-7 of the logits,
     which f32 operands and sums over K / 32 blocks keep (about 2e-7) and
     activations of two bf16 halves do not (2.3e-6 at any K)."""
     print(f"packed head q{bits} K {hidden} rows {rows}", flush=True)
-    cfg = synth.llama_config(1, hidden, 2, 2, 64, 515, head_dim=32)
-    tensors = synth.make_tensors(cfg, 9, "f32", std=0.05)
+    cfg = synth.llama_config(1, hidden, 2, 2, 64, vocab, head_dim=32)
+    tensors = synth.make_tensors(cfg, 9, "f32", std=0.05, fast=vocab > 60000)
     for name in ("self_attn.o_proj", "mlp.down_proj"):
         tensors[f"model.layers.0.{name}.weight"][0][:] = 0
     art = quant.convert_artifact(tensors, bits)
     deq = quant.dequantized_model(art, {n: a.shape for n, (a, _) in tensors.items()}, bits)
     model = DecoderModel.from_bytes(cfg, st.dump(art), f"q{bits}-block32")
-    ids = synth.uniform_ids(rows, rows, 515)
+    ids = synth.uniform_ids(rows, rows, vocab)
     x = np.asarray(deq["model.embed_tokens.weight"][0], np.float64)[ids]
     x = x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-5) * np.asarray(deq["model.norm.weight"][0], np.float64)
     want = x @ np.asarray(deq["lm_head.weight"][0], np.float64).T
@@ -140,6 +195,20 @@ def test_bf16_few_rows(hidden, ffn, heads, kv_heads, rows):
     tensors = synth.make_tensors(cfg, 9, "bf16", std=0.02 if wide else 0.05, fast=wide)
     ref = oracle.OracleModel(cfg, tensors)
     _rows_match(DecoderModel.from_bytes(cfg, st.dump(tensors), "bf16"), ref, 131, rows, 1e-4)
+
+
+# a head of 65500 columns fills two blocks per CU without k splits, so each row
+# form's resident keys (4 rows: 2048, 8: 1024, 16: 512) are refilled, with 128
+@pytest.mark.parametrize("hidden,rows", [(2176, 2), (2176, 4), (1152, 5), (1152, 8), (640, 9), (640, 15)])
+def test_bf16_few_rows_refill_their_activations(hidden, rows):
+    """The few-row form over a k range longer than its resident activations:
+    1e-4 of the row's magnitude."""
+    print(f"bf16 refill rows {rows} K {hidden}", flush=True)
+    cfg = synth.llama_config(1, hidden, hidden // 64, hidden // 64, 256, 65500, head_dim=64,
+                             extra={"tie_word_embeddings": True})
+    tensors = synth.make_tensors(cfg, 9, "bf16", std=0.05, fast=True)
+    ref = oracle.OracleModel(cfg, tensors)
+    _rows_match(DecoderModel.from_bytes(cfg, st.dump(tensors), "bf16"), ref, 65500, rows, 1e-4)
 
 
 # rows per expert on average: 1, 3, 8, 20, 48 and past each
