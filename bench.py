@@ -481,7 +481,7 @@ def c3_packed_bench(bits: int) -> dict:
     t_dec = (t80 - t16) / 64
     greedy_self_check(model, kv, prompt, dev["ids"])
     db = packed_decode_bytes(cfg, 4064 + 48, bits)
-    # 2048-token prefill: doubled-K bf16 projections on the matrix cores
+    # 2048-token prefill: the packed bytes multiplied on the matrix cores
     kvp = model.new_cache(1, 2048 + 8)
     t_pre = []
     for _ in range(3):

@@ -87,8 +87,8 @@ __global__ void __launch_bounds__(256) rmsnorm_k(const float *x, const float *ga
 //   NB_COMBINE x[m] += the routed experts' outputs (CombineArgs), before the
 //             next layer's input norm
 // Measured at H 4096, four rows: plain 12.8 -> 4.7 us (was one wave per row),
-// resid 9.2 -> 5.6 us (was 256 threads, a trip per quarter row), embedding and
-// norm 23.4 -> 6.3 us; 2048 rows: resid 32.6 -> 31.7, embedding and norm 43.5
+// resid of eight splits 9.2 -> 5.5 us (was 256 threads, a trip per quarter row;
+// 16 splits 6.9), embedding and norm 23.4 -> 4.5 us; 2048 rows: resid 32.6 -> 31.7, embedding and norm 43.5
 // -> 26.9 us. H 2048, six rows of two experts: split sums' reduction, combine
 // and norm 3.7 + 6.3 + 4.6 -> 5.3 us.
 enum { NB_PLAIN = 0, NB_RESID = 1, NB_EMBED = 2, NB_COMBINE = 3 };

@@ -1070,8 +1070,11 @@ int attn_decode_splits(int hd, int nkv, int G, int M, int max_t, int *split_len)
     int ns = (int)((target + base - 1) / base);
     ns = std::min(ns, (max_t + step - 1) / step);
     // up to 128 keys of one row: one split, whose keys are all in flight at
-    // once; merging two costs more than the steps it saves (33 - 64 keys of the
-    // tiny decoder: 6.35 -> 4.07 us)
+    // once; merging two to four costs more than the steps it saves. us with
+    // events around the launch, splits -> one: 34, 65 and 128 keys of the tiny
+    // decoder 9.3 -> 7.1, 9.2 -> 7.6, 9.2 -> 7.7, of the 1B shape (8 kv heads,
+    // hd 64, f16 cache) 11.5 -> 9.5, 11.4 -> 10.2, 11.9 -> 10.7, of the 8B shape
+    // (hd 128, f32) 12.8 -> 10.3, 13.1 -> 11.2, 12.8 -> 12.7
     if (M == 1 && max_t <= 128) ns = 1;
     ns = std::max(1, std::min(ns, ATT_MAX_SPLIT));
     int len = (max_t + ns - 1) / ns;

@@ -9,10 +9,11 @@
 // global -> registers a group of 128 keys ahead: 256 contiguous bytes of each
 // row, used at once, in the B-operand layout of v_mfma_f32_16x16x32_bf16.
 // Fewer rows leave room for longer chunks (4 rows: 2048 keys), so the waves
-// meet less often. Bound by HBM: 8B-shape gate/up (235 MB) at 4 rows 55 -> 48.6
-// us (4.8 TB/s; before: 64-row tiles that met at every 32-key stage), o 10.1,
-// down 27, q/k/v 13.3; eight experts of 2048 x 7168 over 12 rows: gate/up 105
-// -> 81, down 90 -> 36 us (before: 128-row tiles, down unsplit).
+// meet less often. Bound by HBM (kernel traces): 8B-shape gate/up (235 MB) at 4
+// rows 55 -> 47.1 us (5.0 TB/s; before: 64-row tiles that met at every 32-key
+// stage), down 24.8, q/k/v 13.7; experts of 2048 x 7168 that six tokens reach,
+// two each: gate/up 77 - 102 us, down 41 - 45 by the number of experts hit
+// (before: 128-row tiles, down unsplit; one layer's products 239 -> 163).
 #include "common.hpp"
 #include "dev.hpp"
 #include "kernels_extra.hpp"
@@ -192,10 +193,14 @@ static bool dense_rows(const GemmArgs &a) {
     return rounds > 0 || (nb == 2 && rounds < 0) || (long long)nb * a.N * a.K * 2 >= 96000000;
 }
 
-// Rows per tile; 0: not this form. Dense launches of at most 15 rows (a
-// decoding batch or forced span of 16 rows and more has a form of its own:
-// gemm_skinny_k, gemm_lds_k); grouped launches of up to 48 rows per group on
-// average, whose groups' weights are read once per tile.
+// Rows per tile; 0: not this form. Dense launches of at most 15 rows (from 16
+// on gemm_skinny_k and gemm_lds_k serve; 16 rows would gain here as well, 8B
+// shape, two layers, 332 -> 314 us, and are not taken). Grouped launches of up
+// to 48 rows per group on average, whose groups' weights are read once per
+// tile: past 64 rows a second tile reads them again. Products of a layer of
+// eight experts, us, wide tiles -> here, rows spread over the experts / all on
+// two of them: 24 per expert 270 -> 248 / 166 -> 133, 48 295 -> 273 / 213 ->
+// 209, 56 299 -> 328 / 220 -> 227, 100 344 -> 445 / 314 -> 382.
 static int rows_tile(const GemmArgs &a) {
     if (a.K % GR_GK) return 0;
     if (!a.grp_offs) return a.M >= 16 || !dense_rows(a) ? 0 : a.M <= 4 ? 4 : a.M <= 8 ? 8 : 16;

@@ -2,8 +2,9 @@
 
 THIS IS THE PARITY CHECKER, NOT THE PRODUCT. Only tests/ and bench.py's
 cpu_baseline leg import it. The product reads packed artifacts in
-esp_amd/csrc/runtime.cpp and dequantizes in the decode GEMV
-(esp_amd/csrc/decode_dev.hpp) and dequant_k (esp_amd/csrc/k_moe.hip).
+esp_amd/csrc/runtime.cpp and multiplies the packed bytes, block scales apart,
+in the decode GEMV (esp_amd/csrc/decode_dev.hpp) and the matrix-core products
+(esp_amd/csrc/k_gemm_packed.hip).
 
 Restates crates/esp/src/infer/decoder/weight_format.rs:
   quantize_projection  weight_format.rs:150-183 (per 32-input block of each

@@ -93,9 +93,9 @@ def test_packed_artifact_refusals():
 @pytest.mark.parametrize("bits", [8, 4])
 @pytest.mark.parametrize("n", [40, 1100])
 def test_packed_prefill_blocks_match_oracle(bits, n):
-    """Prefill of 16+ rows (tiled MFMA attention) and of 1024+ rows (the
-    LDS-streamed GEMM form): packed projections in doubled-K bf16 form on
-    the matrix cores, logits within 1e-4 of the row's largest magnitude."""
+    """Prefill of 40 rows (tiled MFMA attention, the packed products of up to
+    64 rows) and of 1100 (the tiled packed products): logits within 1e-4 of
+    the row's largest magnitude."""
     print(f"bits {bits} rows {n}", flush=True)
     cfg, art, ref = _case(bits, False, seed=9)
     model = DecoderModel.from_bytes(cfg, st.dump(art), FMT[bits])
@@ -108,9 +108,9 @@ def test_packed_prefill_blocks_match_oracle(bits, n):
 
 @pytest.mark.parametrize("bits", [8, 4])
 def test_packed_prefill_split_k_matches_oracle(bits):
-    """1100 rows at hidden 1024 / FFN 2048: the doubled-K projections split
-    K (four splits for down_proj, two for gate/up), so whole splits fall in
-    the second half of the doubled K, where the lo products are skipped."""
+    """1100 rows at hidden 1024 / FFN 2048: on 256 CUs q/k/v and o_proj split K
+    in four, down_proj in six of 352 keys with a last one of 288; gate/up
+    stays whole."""
     print(f"bits {bits} split-K packed prefill", flush=True)
     cfg = synth.llama_config(2, 1024, 8, 2, 2048, 300, head_dim=128)
     tensors = synth.make_tensors(cfg, 9, "f32", std=0.05)
