@@ -1,14 +1,14 @@
 """Benchmark: llama-family decode & prefill tokens/s on one MI355X.
 
-Headline workload ("C3"): Llama-3-8B-shape
-decoder, bf16 weights (random init N(0, 0.02), synthetic) with rank-16 LoRA
-(alpha 32) on q_proj and v_proj, batch 1: a 4064-token uniform-random prompt
-then 64 greedy decode steps, i.e. decode at 4064-4128 (mean 4096) context.
-One "step" is that whole request; `value` is decode tokens/s (the prompt's
-prefill, timed separately, is subtracted). A separate 2048-token prefill is
-reported as prefill tokens/s and a fraction of bf16 MFMA peak.
+Headline workload ("C3"): Llama-3-8B-shape decoder, bf16 weights (random init
+N(0, 0.02), synthetic) with rank-16 LoRA (alpha 32) on q_proj and v_proj, batch
+1: a 4064-token uniform-random prompt then 64 greedy decode steps, i.e. decode
+at 4064-4128 (mean 4096) context. One "step" is that whole request; `value` is
+decode tokens/s (the prompt's prefill, timed separately, is subtracted). A
+separate 2048-token prefill is reported as prefill tokens/s and a fraction of
+bf16 MFMA peak.
 
-`decode_hbm_frac` counts BASELINE.md's algorithmic bytes per token (every
+`decode_hbm_frac` counts the algorithmic bytes per token (every
 weight once in bf16 + the K/V cache once at 2 bytes per element); the
 `roofline` object describes the dominant decode kernel (the SwiGLU gate/up
 GEMV) from HIP events recorded on the KV handle's stream around every launch
@@ -16,7 +16,7 @@ of that kernel in an eager pass; `traffic` is its measured HBM bytes per
 launch from the committed FETCH_SIZE / WRITE_SIZE counter summary.
 `cpu_baseline` times the CPU restatement of esp's burn-ndarray path
 (oracle/) on the same C3 decode at 4096 context on all host cores. The
-other BASELINE configs (C2, C4, C5) and the widened rows are extra objects.
+other workloads (C2, C4, C5) and the widened rows are extra objects.
 """
 from __future__ import annotations
 
@@ -131,7 +131,7 @@ def decode_bytes(cfg, ctx: int, kv_bytes_per_elem: int = 2, lora_rank: int = 0,
                  lora_targets=()) -> dict:
     """Algorithmic HBM bytes of one batch-1 decode step at context `ctx`:
     every weight once (bf16) + the K/V cache once (kv_bytes_per_elem bytes
-    per element; BASELINE.md counts 2) + LoRA A/B (bf16)."""
+    per element; the headline counts 2) + LoRA A/B (bf16)."""
     H, L, F, V = cfg.hidden_size, cfg.num_hidden_layers, cfg.intermediate_size, cfg.vocab_size
     qw, kvw = cfg.query_width(), cfg.kv_heads() * cfg.head_dim()
     lora = 0
@@ -298,7 +298,7 @@ def cpu_baseline(cfg, ctx: int = 4096, decode_runs: int = 7, prefill_len: int = 
 
 
 def c3_headline(steps: int, warmup: int) -> dict:
-    """Llama-3-8B shape bf16 with rank-16 LoRA (alpha 32)
+    """C3: Llama-3-8B shape bf16 with rank-16 LoRA (alpha 32)
     on q_proj and v_proj. One step = one request: a 4064-token prompt and 64
     greedy decode tokens through the device loop (one captured decode step
     replayed per token); decode time = step time minus the prompt's prefill
@@ -397,7 +397,7 @@ def kernel_trace_frac(cfg) -> dict:
 
 
 def c2_bench(steps: int, warmup: int, prompt_len: int = 512, n_decode: int = 256) -> dict:
-    """Llama-3.2-1B shape bf16, batch 1: a 512-token
+    """C2: Llama-3.2-1B shape bf16, batch 1: a 512-token
     prompt then 256 greedy decode steps (device loop); decode tokens/s with
     the prefill subtracted, and the prefill rate."""
     from esp_amd import DecoderModel
@@ -431,7 +431,7 @@ def c2_bench(steps: int, warmup: int, prompt_len: int = 512, n_decode: int = 256
     db = decode_bytes(cfg, prompt_len + n_decode // 2)
     model.close()
     return {"workload": "C2: Llama-3.2-1B shape bf16, 512-token prefill + 256 greedy decode "
-                        "steps, batch 1 (BASELINE configs[1])",
+                        "steps, batch 1",
             "decode_tokens_per_s": round(1.0 / t_dec, 2),
             "decode_ms_per_token": round(t_dec * 1e3, 4),
             "decode_hbm_frac": round(db["total"] / t_dec / 1e9 / HBM_PEAK_GBS, 4),
@@ -635,7 +635,7 @@ def moe_decode_bytes(cfg, ctx: int) -> int:
     """Algorithmic HBM bytes of one batch-1 MoE decode step: attention
     weights, router and the top-k experts' gate/up/down rows of every layer
     (bf16), the head (bf16) and the K/V cache once (2 bytes per element, as
-    BASELINE.md counts it)."""
+    for the headline)."""
     H, L, V = cfg.hidden_size, cfg.num_hidden_layers, cfg.vocab_size
     qw, kvw = cfg.query_width(), cfg.kv_heads() * cfg.head_dim()
     m = cfg.moe
@@ -657,7 +657,7 @@ def moe_prefill_flops(cfg, S: int) -> float:
 
 
 def c4_bench(steps: int) -> dict:
-    """Mixtral-style MoE stack (4 layers, hidden 4096,
+    """C4: Mixtral-style MoE stack (4 layers, hidden 4096,
     8 experts of SwiGLU 14336, top-2 softmax router, vocab 32000), bf16,
     synthetic N(0, 0.02) weights: a 2048-token uniform-random prefill, then
     batch-1 greedy decode at ~2048 context (device loop, captured step)."""
@@ -692,8 +692,7 @@ def c4_bench(steps: int) -> dict:
     db = moe_decode_bytes(cfg, 2048 + n_dec // 2)
     fl = moe_prefill_flops(cfg, 2048)
     res = {"workload": "C4: Mixtral-style MoE (4 layers, hidden 4096, 8 experts x SwiGLU 14336, "
-                       "top-2), bf16; 2048-token prefill, batch-1 decode at 2048-2112 context "
-                       "(BASELINE configs[3])",
+                       "top-2), bf16; 2048-token prefill, batch-1 decode at 2048-2112 context",
            "decode_tokens_per_s": round(1.0 / t_dec, 2),
            "decode_ms_per_token": round(t_dec * 1e3, 4),
            "decode_hbm_frac": round(db / t_dec / 1e9 / HBM_PEAK_GBS, 4),
@@ -706,7 +705,7 @@ def c4_bench(steps: int) -> dict:
 
 
 def c5_bench(steps: int, warmup: int = 2, kv_dtype: str = "f32") -> dict:
-    """constrained decode on the 1B shape, 64 concurrent
+    """C5: constrained decode on the 1B shape, 64 concurrent
     sequences at ~1024 context. Each step: every sequence whose index is
     congruent to the step mod 8 evaluates a forced 8-token block (a causal
     mini-prefill over its warm cache), the other 56 one decode token; then
@@ -772,7 +771,7 @@ def c5_bench(steps: int, warmup: int = 2, kv_dtype: str = "f32") -> dict:
     step_bytes = decode_bytes(cfg, 0)["gemv_weights"] + B * ctx_mid * qkv_kv + 2 * B * V * 4 + B * words * 4
     res = {"workload": "C5: 1B shape bf16, 64 sequences at 1024-1200 context; per step 56 decode "
                        "rows + 8 forced 8-token blocks, allowed-token bitmask (5%) + seeded "
-                       "temperature 0.8 / top-p 0.9 sampling (BASELINE configs[4])",
+                       "temperature 0.8 / top-p 0.9 sampling",
            "sequence_tokens_per_s": round(B * steps / el, 1),
            "rows_per_s": round(rows / el, 1),
            "ms_per_step": round(el / steps * 1e3, 3),
@@ -947,11 +946,11 @@ def main():
                 "uniform-random prompt ids)",
         "config": {"workload": "C3: Llama-3-8B shape bf16 + LoRA r16 alpha 32 on q/v; 4064-token "
                                "prompt then 64 greedy decode steps (decode at 4064-4128 context), "
-                               "batch 1; separate 2048-token prefill (BASELINE configs[2])",
+                               "batch 1; separate 2048-token prefill",
                    "global_batch": 1, "seq_len": 4128, "parallelism": "none (1 GPU)"},
     }
     result.update({k: v for k, v in h.items() if k not in ("value", "ms_per_step")})
-    print(f"c3: decode {h['value']} tok/s ({h['decode_hbm_frac']} of HBM on BASELINE bytes), "
+    print(f"c3: decode {h['value']} tok/s ({h['decode_hbm_frac']} of HBM on algorithmic bytes), "
           f"prefill {h['prefill_tokens_per_s']} tok/s", file=sys.stderr, flush=True)
     legs = [("c2", lambda: c2_bench(steps, args.warmup)), ("c4", lambda: c4_bench(steps)),
             ("c5", lambda: c5_bench(16)), ("c5_grammar", lambda: c5_grammar_bench(32))]

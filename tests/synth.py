@@ -153,7 +153,7 @@ def tiny_llama_case(seed: int, layers: int, hidden: int, heads: int, kv_heads: i
     return cfg, tensors, blob, prompt
 
 
-# BASELINE.json configs[0] (C1): tiny llama, fp32, N(0, 0.02), 2 layers,
+# C1: tiny llama, fp32, N(0, 0.02), 2 layers,
 # hidden 256, 4 heads (hd 64), ffn 688, eps 1e-5, theta 1e4, vocab 1024;
 # 32-token prompt then 32 greedy steps.
 def c1_case(seed: int = 2026):

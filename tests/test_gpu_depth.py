@@ -1,7 +1,7 @@
-"""HIP path vs the CPU oracle at the full depth of BASELINE configs[1] and
-every layer of the 1B shape (16) and of the 8B shape with its
-LoRA (32), prompt prefill then decode steps, logits within the north star's
-bf16 tolerance |a - b| <= 1e-2 + 2e-2 |b| of the oracle's f32 corridor.
+"""HIP path vs the CPU oracle at full depth: every layer of the 1B shape (16)
+and of the 8B shape with its LoRA (32), prompt prefill then decode steps,
+logits within the bf16 tolerance |a - b| <= 1e-2 + 2e-2 |b| of the oracle's f32
+corridor.
 
 Depth matters for the cache's precision: error from rounding keys and
 values grows with the layers it passes through. The default f32 cache is

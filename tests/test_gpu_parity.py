@@ -16,7 +16,7 @@ REF = json.load(open(os.path.join(ARCH, "reference.json")))
 
 
 def _close_bf16(got, want):
-    """bf16 configs: |a - b| <= 1e-2 + 2e-2 |b|."""
+    """bf16 models: |a - b| <= 1e-2 + 2e-2 |b|."""
     return np.all(np.abs(got - want) <= 1e-2 + 2e-2 * np.abs(want))
 
 
@@ -43,7 +43,7 @@ def test_arch_golden(case):
 
 
 def test_c1_fp32_greedy_matches_oracle():
-    """32-token prompt, 32 greedy steps; ids bit-exact,
+    """C1: 32-token prompt, 32 greedy steps; ids bit-exact,
     logits within 1e-4 relative (to the row's max magnitude)."""
     cfg, tensors, blob, prompt = synth.c1_case()
     model = DecoderModel.from_bytes(cfg, blob, "f32")
@@ -404,7 +404,7 @@ def test_bf16_long_context_decode_splits(kv_dtype):
 
 def _adapter(cfg, rank, targets, seed, fmt):
     """PEFT LoRA tensors base_model.model.model.layers.{i}.self_attn.{m}.lora_{A,B}.weight,
-    A ~ N(0, 0.02), B ~ N(0, 0.01) (BASELINE configs[2])."""
+    A ~ N(0, 0.02), B ~ N(0, 0.01)."""
     H, qw, kvw = cfg.hidden_size, cfg.query_width(), cfg.kv_heads() * cfg.head_dim()
     out = {}
     for l in range(cfg.num_hidden_layers):

@@ -1,4 +1,5 @@
-"""HIP path vs the CPU oracle at the full widths of BASELINE configs[2..4].
+"""HIP path vs the CPU oracle at full width: the 8B shape, the routed stack and
+the 1B shape.
 
 Depth is sliced to two layers (the per-layer kernels are the same at every
 depth); every width is the config's own: hidden, heads, head_dim, ffn,
@@ -7,7 +8,7 @@ times at these shapes (decode GEMVs at hidden 4096 with K up to 14336,
 routed-expert decode, the 64-row sampler over 128256 tokens), so the bench
 figures come from checked code.
 
-Tolerances are the north star's for bf16 configs: |a - b| <= 1e-2 + 2e-2|b|
+Tolerances are those of bf16 models: |a - b| <= 1e-2 + 2e-2|b|
 against the oracle's f32 corridor; sampled ids, RNG states and masks are
 bit-exact against the oracle run on the device's own logits.
 """
@@ -35,8 +36,7 @@ def _err(got, want):
 
 
 def _lora(cfg, seed):
-    """PEFT r16 alpha 32 on q_proj / v_proj, A ~ N(0, 0.02), B ~ N(0, 0.01)
-    (BASELINE configs[2])."""
+    """PEFT r16 alpha 32 on q_proj / v_proj, A ~ N(0, 0.02), B ~ N(0, 0.01)."""
     H, qw, kvw = cfg.hidden_size, cfg.query_width(), cfg.kv_heads() * cfg.head_dim()
     out = {}
     for l in range(cfg.num_hidden_layers):
