@@ -178,16 +178,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ROWS <
 
 // Dense launches (2 - 15 rows) that the skinny streamed form, 128 columns and
 // one k range a block, does not do better. Where its blocks fill one round of
-// the CUs or less it keeps up: a block's whole range is then in flight from
-// the start. Past one round the last round is ragged; gate/up below a round
-// gets twice the blocks here; and from 96 MB on the resident activations pay.
-// us per launch (events around it), skinny -> here, at 2 and 14 rows: o of the 1B shape (128
-// blocks) 7.9 -> 7.9, 8.1 -> 8.9, its gate/up (256, 67 MB) 20.2 -> 20.0, 21.4 ->
-// 22.9, down (256, 34 MB) 12.9 -> 13.6, 13.0 -> 15.2; 8B-shape q/k/v (384
-// blocks) 19.0 -> 15.4, 19.4 -> 17.5, gate/up (448) 61.7 -> 53.6, 62.8 -> 58.4,
-// down (256, 117 MB) 32.4 -> 29.7, 34.9 -> 33.0; gate/up of 1024 x 2816 (88)
-// 13.6 -> 11.4, 14.0 -> 12.5; gate/up of 3072 x 8192 (256, 101 MB) 33 -> 28, 33.3
-// -> 31.6.
+// the CUs or less it keeps up: a block's whole range is then in flight from the
+// start. Past one round the last round is ragged; gate/up below a round gets
+// twice the blocks here; and from 96 MB on the resident activations pay. us per
+// launch (events around it), skinny -> here, at 2 and 14 rows: o of the 1B
+// shape (128 blocks) 7.9 -> 7.9, 8.1 -> 8.9, its gate/up (256, 67 MB) 20.2 ->
+// 20.0, 21.4 -> 22.9, down (256, 34 MB) 12.9 -> 13.6, 13.0 -> 15.2; 8B-shape
+// q/k/v (384 blocks) 19.0 -> 15.4, 19.4 -> 17.5, gate/up (448) 61.7 -> 53.6,
+// 62.8 -> 58.4, down (256, 117 MB) 32.4 -> 29.7, 34.9 -> 33.0; gate/up of 1024
+// x 2816 (88) 13.6 -> 11.4, 14.0 -> 12.5; gate/up of 3072 x 8192 (256, 101 MB)
+// 33 -> 28, 33.3 -> 31.6.
 static bool dense_rows(const GemmArgs &a) {
     const int nb = a.w2 ? 2 : 1, rounds = gemm_skinny_rounds(a);
     return rounds > 0 || (nb == 2 && rounds < 0) || (long long)nb * a.N * a.K * 2 >= 96000000;
